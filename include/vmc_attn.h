@@ -107,7 +107,11 @@ int vmc_convert_fp8(void* dst_cache, const void* src_cache, double scale, int64_
  * Limits: head_dim 64, 128 or 256; block_size 16 at head_dim 128.  At
  * head_dim 128 with num_kv_heads <= 8 and num_heads / num_kv_heads <= 16 the
  * tuned kernel runs: two launches on `stream` (split pass, merge of cut
- * sequences).  Other head dims and head counts run a one-wave-per-row kernel
+ * sequences).  head_dim 64 and 256 with block_size 16, num_heads /
+ * num_kv_heads <= 16, 16-byte aligned operands and f16 / bf16 pages of
+ * q_dtype or GGUF pages run the MFMA decode: the same two launches where the
+ * workspace has room for partial rows, else one pass per sequence.  Other
+ * shapes run a one-wave-per-row kernel
  * (one launch, no workspace).  No host synchronisation.  The workspace size
  * depends on the current device's CU count.
  */

@@ -438,6 +438,111 @@ __global__ void __launch_bounds__(1024) decode_merge_kernel(DecodeParams p) {
     *reinterpret_cast<u32x4*>(orow + 8 * r16) = u32x4{w4[0], w4[1], w4[2], w4[3]};
 }
 
+// The same combination over rows of D + 4 floats, four waves per (sequence,
+// query head): grid (B, Hq), 256 threads; wave w takes pieces w, w + 4, ...
+// (sixteen rows in flight, so 64 pieces cost one round of loads), lane l dims
+// l D / 64 .. ; the four partial sums meet in LDS.
+template <int D>
+__global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) {
+    constexpr int NV = D / 64;
+    typedef float fv __attribute__((ext_vector_type(NV)));
+    __shared__ __attribute__((aligned(16))) float red[4][D + 4];
+    const int b = blockIdx.x, hq = blockIdx.y;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int carry = 0, ps_b = 0, pg_b = 0;
+    for (int b0 = 0; b0 < p.B; b0 += 64) {
+        int L = 0;
+        const int pg = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
+        const int incl = wave_incl_scan(pg, lane);
+        if (b >= b0 && b < b0 + 64) {  // uniform over the wave
+            ps_b = __shfl(carry + incl - pg, b - b0, 64);
+            pg_b = __shfl(pg, b - b0, 64);
+        }
+        carry += __shfl(incl, 63, 64);
+    }
+    const int T = carry;
+    uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + ((int64_t)b * p.Hq + hq) * D + NV * lane;
+    auto put = [&](const fv& x) __attribute__((always_inline)) {
+        uint16_t h[NV];
+#pragma unroll
+        for (int e = 0; e < NV; ++e) h[e] = p.q_bf16 ? f32_to_bf16_bits(x[e]) : f32_to_f16_bits(x[e]);
+        if constexpr (NV == 4)
+            *reinterpret_cast<u32x2*>(orow) = u32x2{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16)};
+        else if constexpr (NV == 2)
+            *reinterpret_cast<uint32_t*>(orow) = h[0] | ((uint32_t)h[1] << 16);
+        else
+            orow[0] = h[0];
+    };
+    if (pg_b == 0) {
+        if (wave == 0) put(fv(0.0f));
+        return;
+    }
+    const int n = effective_wgs(p, T, p.grid);
+    const int w0 = wg_of_page(ps_b, n, T), w1 = wg_of_page(ps_b + pg_b - 1, n, T);
+    if (w0 == w1) return;  // written by its range
+    const int nseg = w1 - w0 + 1;
+    const int64_t rs = (int64_t)p.Hq * (D + 4);
+    auto row = [&](int s) {  // piece s = range w0 + s
+        const int64_t slot = s == 0 ? 2 * w0 + 1 : 2 * (w0 + s);
+        return p.part + slot * rs + (int64_t)hq * (D + 4);
+    };
+    float M = kNegInf, L = 0.0f;
+    fv acc = fv(0.0f);
+    for (int s0 = wave; s0 < nseg; s0 += 64) {
+        fv o[16];
+        float2 ml[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const float* r = row(min(s0 + 4 * u, nseg - 1));
+            ml[u] = *reinterpret_cast<const float2*>(r + D);
+            o[u] = *reinterpret_cast<const fv*>(r + NV * lane);
+        }
+        float mx = M;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) mx = s0 + 4 * u < nseg ? fmaxf(mx, ml[u].x) : mx;
+        if (mx > M && M != kNegInf) {  // wave-uniform
+            const float f = __builtin_amdgcn_exp2f(M - mx);
+            L *= f;
+#pragma unroll
+            for (int e = 0; e < NV; ++e) acc[e] *= f;
+        }
+        M = mx;
+        const float Mu = M == kNegInf ? 0.0f : M;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const float wu = s0 + 4 * u < nseg ? __builtin_amdgcn_exp2f(ml[u].x - Mu) : 0.0f;
+            L = __builtin_fmaf(ml[u].y, wu, L);
+#pragma unroll
+            for (int e = 0; e < NV; ++e) acc[e] = __builtin_fmaf(o[u][e], wu, acc[e]);
+        }
+    }
+    *reinterpret_cast<fv*>(&red[wave][NV * lane]) = acc;
+    if (lane == 0) {
+        red[wave][D] = M;
+        red[wave][D + 1] = L;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float Mg = kNegInf;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) Mg = fmaxf(Mg, red[w][D]);
+    const float Mgu = Mg == kNegInf ? 0.0f : Mg;
+    float Lg = 0.0f;
+    fv og = fv(0.0f);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float f = red[w][D] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(red[w][D] - Mgu);
+        Lg = __builtin_fmaf(red[w][D + 1], f, Lg);
+        const fv v = *reinterpret_cast<const fv*>(&red[w][NV * lane]);
+#pragma unroll
+        for (int e = 0; e < NV; ++e) og[e] = __builtin_fmaf(v[e], f, og[e]);
+    }
+    const float inv = Lg > 0.0f ? 1.0f / Lg : 0.0f;
+#pragma unroll
+    for (int e = 0; e < NV; ++e) og[e] *= inv;
+    put(og);
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------ host

@@ -41,6 +41,7 @@
 #include "decode_plan.hpp"
 #include "generic_attn.hpp"
 #include "kv_quant.hpp"
+#include "paged_decode_hd.hpp"
 #include "prefill_api.hpp"
 
 #include <mutex>
@@ -1430,8 +1431,10 @@ int paged_decode_rows(void* out, const void* query, const void* key_cache, const
                       int q_dtype, int kv_format, int layout, int max_num_kv_splits, void* workspace,
                       size_t workspace_bytes, vmc_stream_t stream) {
     if (generic_head_dim(head_dim) || beyond_tuned_decode(head_dim, num_heads, num_kv_heads)) {
-        // head_dim 64 / 256, and head counts past the tuned kernels' (see
-        // beyond_tuned_decode): one wave per (row, query head), no workspace
+        // head_dim 64 / 256 (paged_decode_hd.hip where paged_decode_hd_takes,
+        // else one wave per (row, query head)), and head counts past the tuned
+        // kernels' (beyond_tuned_decode: one wave per (row, query head)).  A
+        // workspace is used where there is one, not required
         if (batch_size < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 ||
             block_size <= 0 || max_num_blocks_per_req <= 0)
             return VMC_EINVAL;
@@ -1463,6 +1466,9 @@ int paged_decode_rows(void* out, const void* query, const void* key_cache, const
         a.Hkv = num_kv_heads;
         a.D = head_dim;
         a.scale = scale;
+        if (paged_decode_hd_takes(a))
+            return paged_decode_hd(a, max_num_kv_splits, workspace, workspace_bytes,
+                                   reinterpret_cast<hipStream_t>(stream));
         return gen_attention(a, reinterpret_cast<hipStream_t>(stream));
     }
     DecodeParams prm = {};

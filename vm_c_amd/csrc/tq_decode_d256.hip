@@ -572,106 +572,6 @@ __global__ void __launch_bounds__(512, 1) tq_decode_d256_kernel(DecodeParams p) 
     }
 }
 
-// Combines the pieces of sequences cut by range boundaries (head_dim 256):
-// decode_merge_kernel's rule over rows of kPartRow2 floats (o unnormalised, m,
-// l).  Grid (B, Hq), 4 waves per (sequence, query head): wave w takes pieces
-// w, w + 4, ... (sixteen rows in flight), lane l dims 4 l .. + 3; the four
-// partial sums are combined through LDS.
-__global__ void __launch_bounds__(256) decode_merge_d256_kernel(DecodeParams p) {
-    __shared__ __attribute__((aligned(16))) float red[4][kD2 + 4];  // rows 16-byte aligned
-    const int b = blockIdx.x, hq = blockIdx.y;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int carry = 0, ps_b = 0, pg_b = 0;
-    for (int b0 = 0; b0 < p.B; b0 += 64) {
-        int L = 0;
-        const int pg = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
-        const int incl = wave_incl_scan(pg, lane);
-        if (b >= b0 && b < b0 + 64) {  // uniform over the wave
-            ps_b = __shfl(carry + incl - pg, b - b0, 64);
-            pg_b = __shfl(pg, b - b0, 64);
-        }
-        carry += __shfl(incl, 63, 64);
-    }
-    const int T = carry;
-    uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + ((int64_t)b * p.Hq + hq) * kD2;
-    if (pg_b == 0) {
-        if (wave == 0) reinterpret_cast<u32x2*>(orow)[lane] = u32x2{0u, 0u};
-        return;
-    }
-    const int n = effective_wgs(p, T, p.grid);
-    const int w0 = wg_of_page(ps_b, n, T), w1 = wg_of_page(ps_b + pg_b - 1, n, T);
-    if (w0 == w1) return;  // written by its range
-    const int nseg = w1 - w0 + 1;
-    const int64_t rs = (int64_t)p.Hq * kPartRow2;
-    auto row = [&](int s) {  // piece s = range w0 + s
-        const int slot = s == 0 ? 2 * w0 + 1 : 2 * (w0 + s);
-        return p.part + slot * rs + (int64_t)hq * kPartRow2;
-    };
-    float M = kNegInf, L = 0.0f;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = wave; s0 < nseg; s0 += 64) {
-        // (rows are 8-byte aligned: float2 loads)
-        float2 o[16][2], ml[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const float* r = row(min(s0 + 4 * u, nseg - 1));
-            ml[u] = *reinterpret_cast<const float2*>(r + kD2);
-            o[u][0] = *reinterpret_cast<const float2*>(r + 4 * lane);
-            o[u][1] = *reinterpret_cast<const float2*>(r + 4 * lane + 2);
-        }
-        float mx = M;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) mx = s0 + 4 * u < nseg ? fmaxf(mx, ml[u].x) : mx;
-        if (mx > M && M != kNegInf) {  // wave-uniform
-            const float f = __builtin_amdgcn_exp2f(M - mx);
-            L *= f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] *= f;
-        }
-        M = mx;
-        const float Mu = M == kNegInf ? 0.0f : M;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const float wu = s0 + 4 * u < nseg ? __builtin_amdgcn_exp2f(ml[u].x - Mu) : 0.0f;
-            L = __builtin_fmaf(ml[u].y, wu, L);
-            acc[0] = __builtin_fmaf(o[u][0].x, wu, acc[0]);
-            acc[1] = __builtin_fmaf(o[u][0].y, wu, acc[1]);
-            acc[2] = __builtin_fmaf(o[u][1].x, wu, acc[2]);
-            acc[3] = __builtin_fmaf(o[u][1].y, wu, acc[3]);
-        }
-    }
-    *reinterpret_cast<f32x4*>(&red[wave][4 * lane]) = f32x4{acc[0], acc[1], acc[2], acc[3]};
-    if (lane == 0) {
-        red[wave][kD2] = M;
-        red[wave][kD2 + 1] = L;
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    float Mg = kNegInf;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) Mg = fmaxf(Mg, red[w][kD2]);
-    const float Mgu = Mg == kNegInf ? 0.0f : Mg;
-    float Lg = 0.0f;
-    f32x4 og = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const float f = red[w][kD2] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(red[w][kD2] - Mgu);
-        Lg = __builtin_fmaf(red[w][kD2 + 1], f, Lg);
-        const f32x4 v = *reinterpret_cast<const f32x4*>(&red[w][4 * lane]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) og[e] = __builtin_fmaf(v[e], f, og[e]);
-    }
-    const float inv = Lg > 0.0f ? 1.0f / Lg : 0.0f;
-    uint32_t w2[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const uint16_t x0 = p.q_bf16 ? f32_to_bf16_bits(og[2 * e] * inv) : f32_to_f16_bits(og[2 * e] * inv);
-        const uint16_t x1 = p.q_bf16 ? f32_to_bf16_bits(og[2 * e + 1] * inv) : f32_to_f16_bits(og[2 * e + 1] * inv);
-        w2[e] = (uint32_t)x0 | ((uint32_t)x1 << 16);
-    }
-    reinterpret_cast<u32x2*>(orow)[lane] = u32x2{w2[0], w2[1]};
-}
-
 template <int KB, int HK, bool BF>
 int launch_d256(DecodeParams& prm, hipStream_t stream) {
     using DG = D2Geo<KB, HK>;
@@ -684,7 +584,7 @@ int launch_d256(DecodeParams& prm, hipStream_t stream) {
     hipLaunchKernelGGL((tq_decode_d256_kernel<KB, HK, BF>), dim3(nwg), dim3(512), 0, stream, prm);
     VMC_LAUNCH_CHECK();
     if (!prm.per_seq) {
-        hipLaunchKernelGGL(decode_merge_d256_kernel, dim3(prm.B, prm.Hq), dim3(256), 0, stream, prm);
+        hipLaunchKernelGGL(decode_merge_rows_kernel<kD2>, dim3(prm.B, prm.Hq), dim3(256), 0, stream, prm);
         VMC_LAUNCH_CHECK();
     }
     return VMC_OK;
