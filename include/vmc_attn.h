@@ -374,8 +374,10 @@ int vmc_batch_token_rows(int32_t* row_seq, int32_t* row_pos, const int32_t* toke
  * Optional fused quantize-on-append: when key_cache != NULL the same launch
  * writes every K/V row into the paged cache (kv_format/layout as in
  * vmc_reshape_and_cache, slot_mapping int64 [num_tokens]).
- * Limits: head_dim 64, 128 or 256 (64 and 256: a one-wave-per-row kernel,
- * then the append by vmc_reshape_and_cache), num_heads % num_kv_heads == 0.
+ * Limits: head_dim 64, 128 or 256 (64 and 256: the append by
+ * vmc_reshape_and_cache, then the tiled kernel of those sizes, or a
+ * one-wave-per-row kernel where q, out, K or V is not 16-byte aligned),
+ * num_heads % num_kv_heads == 0.
  */
 int vmc_flash_attention_prefill(void* output, const void* query, const void* key,
                                 const void* value, int num_tokens, int num_heads,

@@ -35,6 +35,8 @@
 #include "generic_attn.hpp"
 #include "kv_quant.hpp"
 #include "prefill_api.hpp"
+#include "prefill_dev.hpp"
+#include "prefill_hd.hpp"
 #include "vmc_tq.hpp"
 
 namespace vmc {
@@ -92,45 +94,6 @@ struct PrefillParams {
     const uint8_t* vt_flag;
     int vt_tiles;
 };
-
-template <bool BF16>
-struct MT;
-template <>
-struct MT<true> {
-    using v8 = bf16x8;
-    static __device__ __forceinline__ f32x16 mma(v8 a, v8 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ uint16_t cvt(float x) { return f32_to_bf16_bits(x); }
-    static __device__ __forceinline__ float back(uint16_t b) { return bf16_bits_to_f32(b); }
-};
-template <>
-struct MT<false> {
-    using v8 = f16x8;
-    static __device__ __forceinline__ f32x16 mma(v8 a, v8 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ uint16_t cvt(float x) { return f32_to_f16_bits(x); }
-    static __device__ __forceinline__ float back(uint16_t b) { return f16_bits_to_f32(b); }
-};
-
-template <typename V8>
-__device__ __forceinline__ V8 as_v8(u32x4 w) {
-    return __builtin_bit_cast(V8, w);
-}
-
-// One 16-byte-per-lane load-to-LDS transfer: lane L's 16 bytes from src land
-// at LDS address m0 + 16 L.  Issued from asm so the compiler does not track it: it
-// would otherwise make every later LDS read wait for all transfers in
-// flight (it cannot tell the slots apart); the kernel waits for them itself.
-__device__ __forceinline__ void dma16m(const void* src, uint32_t m0) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(m0) : "memory");
-}
-// The same transfer from a wave-uniform base (SGPRs) plus a 32-bit per-lane
-// offset: no per-lane 64-bit address arithmetic.
-__device__ __forceinline__ void dma16s(const void* base, uint32_t off, uint32_t m0) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
-}
 
 // All LDS of the kernel: the per-wave exchange, the fp16 V^T tiles (128
 // rows of 64 keys, 16-byte chunk i of row d at position i ^ ((d >> 1) & 7)),
@@ -1278,8 +1241,9 @@ int local_prefill(void* output, const void* query, const void* key, const void* 
                   int dtype, void* key_cache, void* value_cache, const int64_t* slot_mapping, int64_t block_size,
                   int kv_format, int layout, void* ws, size_t ws_bytes, vmc_stream_t stream) {
     if (generic_head_dim(head_dim)) {
-        // head_dim 64 / 256: the append by vmc_reshape_and_cache, then one
-        // wave per (token, query head) over this step's K/V
+        // head_dim 64 / 256: the append by vmc_reshape_and_cache, then
+        // prefill_hd.hip, or for operands it does not take one wave per
+        // (token, query head) over this step's K/V
         if (num_tokens < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0)
             return VMC_EINVAL;
         if (dtype != VMC_DTYPE_F16 && dtype != VMC_DTYPE_BF16) return VMC_EINVAL;
@@ -1308,6 +1272,7 @@ int local_prefill(void* output, const void* query, const void* key, const void* 
         a.Hkv = num_kv_heads;
         a.D = head_dim;
         a.scale = scale;
+        if (prefill_hd_takes(a)) return prefill_hd(a, reinterpret_cast<hipStream_t>(stream));
         return gen_attention(a, reinterpret_cast<hipStream_t>(stream));
     }
     if (head_dim != kD || num_tokens < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
