@@ -37,6 +37,7 @@
 #include "prefill_api.hpp"
 #include "prefill_dev.hpp"
 #include "prefill_hd.hpp"
+#include "tq_lut.hpp"
 #include "vmc_tq.hpp"
 
 namespace vmc {
@@ -73,6 +74,8 @@ struct PrefillParams {
     int q_bf16;          // paged: q / out (TurboQuant: and the stored halves) are bf16
     // TurboQuant slots: Lloyd-Max centroids, 1 / sqrt(d), field offsets
     float cent[16];
+    uint32_t sq_plane[12];  // cent[i]^2 / sq_unit, rounded: byte planes (tq_lut.hpp)
+    float sq_unit;
     float rot_c;
     int mse_bytes, key_packed, val_data;
     int norm_corr;  // keys scaled by 1 / ||C[codes]|| (else by the stored norm alone)
@@ -108,7 +111,8 @@ struct PrefillParams {
 struct PrefillLds {
     float scratch[2][NW][32];            // [alpha, l][wave][row]
     alignas(8) uint8_t wide[NSLOT][NW];  // bf16: wave w's V rows of the tile need the exact mode
-    float cent[16];                      // TurboQuant key centroids
+    float tq_base[2][16];                // TurboQuant: key centroids, value codes 0 .. 15
+    uint32_t tq_sq[12];                  // squared centroids, 24-bit fixed point, as byte planes
     alignas(16) uint8_t vtr[NSLOT][kD * BN * 2];  // [slot][dim][kv position] fp16 V^T
     uint8_t tile[NSLOT][2][BN * 256];             // [slot][K, V][row][position]
 };
@@ -255,7 +259,8 @@ prefill_kernel(PrefillParams p) {
                          ((uint32_t)f32_to_f16_bits(y[s][2 * e + 1] * p.rot_c) << 16)) ^ qflip;
             qb[s] = as_v8<V8>(u32x4{wd[0], wd[1], wd[2], wd[3]});
         }
-        if (tid < 16) lds.cent[tid] = p.cent[tid];
+        if (tid < 32) lds.tq_base[tid >> 4][tid & 15] = tid < 16 ? p.cent[tid] : (float)(tid & 15);
+        if (tid < 12) lds.tq_sq[tid] = p.sq_plane[tid];
         __syncthreads();
     }
 
@@ -406,10 +411,95 @@ prefill_kernel(PrefillParams p) {
     auto store_q = [&](auto slot_c) __attribute__((always_inline)) {
         if constexpr (SRC == SRC_Q8 || SRC == SRC_Q4 || kTQ) {
             constexpr int SL = decltype(slot_c)::value;
-            if constexpr (kTQ) {
-                u32x4 kw[4];
+            if constexpr (kTQ && !kK8) {
+                // A row's K (or V) holds at most 8 or 16 distinct fp16 values:
+                // C[i] * norm / ||C[codes]|| (C[i] * norm without the norm
+                // correction), or i * scale + zero.  They are computed once per
+                // lane and block, split into low and high bytes, and looked up
+                // four codes at a time by byte permutes (tq_lut.hpp): 1497 us
+                // on 2048 tokens over a 30720-token prefix of 3-bit slots, where
+                // one LDS gather, multiply and conversion per code took 1687 us.
+                constexpr int NB = TKB > TVB ? TKB : TVB;
+                using Lut = TqLut<NB>;
                 const bool kpart = lane < 32;
-                constexpr int NC = 4 * (TKB > TVB ? TKB : TVB) / 4;  // code dwords
+                uint32_t c[NB];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) c[i] = __builtin_amdgcn_alignbyte(qraw[i + 1], qraw[i], tq_sh);
+                const uint32_t hw2 = qraw[kNC];
+                auto half_f = [&](uint32_t b) {
+                    return qbf ? __builtin_bit_cast(float, b << 16) : f16_bits_to_f32(b & 0xffffu);
+                };
+                // chunk j = codes 8j .. 8j+7; at step j this lane converts
+                // chunk (j + rot) & 3, by two selects on the bits of rot (a
+                // select by the chunk index compiles to divergent branches)
+                const int rot = qr & 3;
+                const bool r0 = (rot & 1) != 0, r1 = (rot & 2) != 0;
+                auto turn = [&](uint32_t (&x)[4]) __attribute__((always_inline)) {
+                    const uint32_t y0 = r0 ? x[1] : x[0], y1 = r0 ? x[2] : x[1];
+                    const uint32_t y2 = r0 ? x[3] : x[2], y3 = r0 ? x[0] : x[3];
+                    x[0] = r1 ? y2 : y0, x[1] = r1 ? y3 : y1, x[2] = r1 ? y0 : y2, x[3] = r1 ? y1 : y3;
+                };
+                uint32_t sel[4][2];
+                {
+                    uint32_t x3[4], x4[4];
+                    if constexpr (TKB == 3) {
+                        tq_chunks<3>(c, x3);
+                        turn(x3);
+                    }
+                    if constexpr (NB == 4) {
+                        tq_chunks<4>(c, x4);
+                        turn(x4);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        uint32_t s3[2] = {}, s4[2] = {};
+                        if constexpr (TKB == 3) tq_spread<3>(x3[j], s3);
+                        if constexpr (NB == 4) tq_spread<4>(x4[j], s4);
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            sel[j][u] = NB == 3 ? s3[u] : TKB == 4 ? s4[u] : kpart ? s3[u] : s4[u];
+                    }
+                }
+                // ||C[codes]||^2 as a sum of 24-bit fixed-point squares (exact
+                // integers; the four lanes of a quad hold the row's four blocks)
+                float f = half_f(hw2), add = 0.0f;
+                {
+                    uint32_t sq[TKB == 4 ? 12 : 6];
+#pragma unroll
+                    for (int i = 0; i < (TKB == 4 ? 12 : 6); ++i) sq[i] = lds.tq_sq[i];
+                    uint32_t ss = 0;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) TqLut<TKB>::add_fixed24(sel[j][u], sq, ss);
+                    ss += (uint32_t)__shfl_xor((int)ss, 1, kWave);
+                    ss += (uint32_t)__shfl_xor((int)ss, 2, kWave);
+                    const float nrm = __builtin_amdgcn_rsqf(__builtin_fmaf((float)ss, p.sq_unit, 1e-16f));
+                    if (kpart) {
+                        f *= p.norm_corr ? nrm : 1.0f;
+                    } else {
+                        add = half_f(hw2 >> 16);
+                    }
+                }
+                Lut lut;
+                {
+                    float base[1 << NB];
+#pragma unroll
+                    for (int i = 0; i < (1 << NB); ++i) base[i] = lds.tq_base[lane >> 5][i];
+                    lut.build(base, f, add);
+                }
+                uint8_t* dst = lds.tile[SL][lane >> 5] + qr * 256;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const u32x2 a = lut.pick(sel[j][0]), b = lut.pick(sel[j][1]);
+                    const u32x4 x = {a[0], a[1], b[0], b[1]};
+                    *reinterpret_cast<u32x4*>(dst + 16 * ((4 * qblk_ + ((j + rot) & 3)) ^ swz(qr))) = x;
+                }
+            } else if constexpr (kK8) {
+                // fp8 keys: each of the lane's 32 bytes is exact in fp16;
+                // V = code * scale + zero
+                u32x4 kw[4];
+                constexpr int NC = 4 * TKB / 4;  // code dwords
                 uint32_t c[NC];
 #pragma unroll
                 for (int i = 0; i < NC; ++i) c[i] = __builtin_amdgcn_alignbyte(qraw[i + 1], qraw[i], tq_sh);
@@ -417,63 +507,26 @@ prefill_kernel(PrefillParams p) {
                 auto half_f = [&](uint32_t b) {
                     return qbf ? __builtin_bit_cast(float, b << 16) : f16_bits_to_f32(b & 0xffffu);
                 };
-                const int bits = kpart ? TKB : TVB;
-                uint32_t code[32];
-#pragma unroll
-                for (int j = 0; j < 32; ++j) {
-                    // 3-bit: code j at bits 3j of c[0..2]; 4-bit: at bits 4j
-                    uint32_t code3 = 0, code4 = 0;
-                    if constexpr (TKB == 3 || TVB == 3) {
-                        const int b0 = 3 * j, wi = b0 >> 5, sh = b0 & 31;
-                        code3 = (sh <= 29 ? (c[wi] >> sh) : __builtin_amdgcn_alignbit(c[wi + 1], c[wi], sh)) & 7u;
-                    }
-                    if constexpr (NC >= 4) code4 = (c[j >> 3] >> (4 * (j & 7))) & 15u;
-                    code[j] = bits == 3 ? code3 : code4;
-                }
-                auto kw_from = [&](const float (&v)[32]) __attribute__((always_inline)) {
+                if (lane < 32) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            kw[j][e] = (uint32_t)f32_to_f16_bits(v[8 * j + 2 * e]) |
-                                       ((uint32_t)f32_to_f16_bits(v[8 * j + 2 * e + 1]) << 16);
-                };
-                float v[32];
-                if (kpart) {
-                    if constexpr (kK8) {
-                        // fp8 keys: each of the lane's 32 bytes is exact in fp16
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const int b = 8 * j + 2 * e;  // bytes b and b + 1 share a word
-                                const uint32_t wv = c[b >> 2] >> (8 * (b & 3));
-                                kw[j][e] = (uint32_t)fp8_f16_bits(wv, p.fp8_e4b15) |
-                                           ((uint32_t)fp8_f16_bits(wv >> 8, p.fp8_e4b15) << 16);
-                            }
-                    } else {
-                        // K = C[code] * norm / ||C[codes]|| over the row's 128 dims
-                        // (C[code] * norm without the norm correction)
-                        // (the four lanes of a quad hold its four blocks)
-                        float ss = 0.0f;
-#pragma unroll
-                        for (int j = 0; j < 32; ++j) {
-                            v[j] = lds.cent[code[j]];
-                            ss = __builtin_fmaf(v[j], v[j], ss);
+                        for (int e = 0; e < 4; ++e) {
+                            const int b = 8 * j + 2 * e;  // bytes b and b + 1 share a word
+                            const uint32_t wv = c[b >> 2] >> (8 * (b & 3));
+                            kw[j][e] = (uint32_t)fp8_f16_bits(wv, p.fp8_e4b15) |
+                                       ((uint32_t)fp8_f16_bits(wv >> 8, p.fp8_e4b15) << 16);
                         }
-                        ss += __shfl_xor(ss, 1, kWave);
-                        ss += __shfl_xor(ss, 2, kWave);
-                        const float f = half_f(hw2) * (p.norm_corr ? __builtin_amdgcn_rsqf(ss + 1e-16f) : 1.0f);
-#pragma unroll
-                        for (int j = 0; j < 32; ++j) v[j] *= f;
-                        kw_from(v);
-                    }
                 } else {
-                    // V = code * scale + zero
                     const float vs = half_f(hw2), vz = half_f(hw2 >> 16);
 #pragma unroll
-                    for (int j = 0; j < 32; ++j) v[j] = __builtin_fmaf((float)code[j], vs, vz);
-                    kw_from(v);
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t b = c[j] >> (8 * e);
+                            kw[j][e] = (uint32_t)f32_to_f16_bits(__builtin_fmaf((float)(b & 15u), vs, vz)) |
+                                       ((uint32_t)f32_to_f16_bits(__builtin_fmaf((float)((b >> 4) & 15u), vs, vz)) << 16);
+                        }
                 }
                 // chunk (j + rot) & 3 at step j, by two selects on the bits
                 // of rot (a select by the chunk index compiles to divergent
@@ -1129,6 +1182,7 @@ int tq_prefill_tiled(void* out, const void* query, const void* kv_cache, const i
     if (!cfg->key_fp8) {
         const TQTables& tab = tq_tables(kD, cfg->key_quant_bits);
         for (int i = 0; i < 16; ++i) prm.cent[i] = i < tab.n_centroids ? tab.centroids[i] : 0.0f;
+        prm.sq_unit = tq_fixed24_planes(prm.cent, cfg->key_quant_bits, prm.sq_plane);
         prm.rot_c = tab.rot_c;
     }
     prm.fp8_e4b15 = cfg->fp8_e4b15 ? 1 : 0;
