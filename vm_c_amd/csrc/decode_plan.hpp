@@ -4,11 +4,11 @@
 // table builder, the merge kernel of cut sequences and the grid sizing.
 #pragma once
 
+#include "device_cus.hpp"
 #include "vmc_common.hpp"
 #include "vmc_tq.hpp"
 
 #include <algorithm>
-#include <mutex>
 #include <utility>
 
 namespace vmc {
@@ -548,20 +548,6 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
 // ------------------------------------------------------------------ host
 
 constexpr int kPpsMin = 2;
-
-inline int num_cus() {
-    static std::mutex mu;
-    static int cached[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    std::lock_guard<std::mutex> lk(mu);
-    if (!cached[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
 
 // Launched workgroups for the flat layout: one resident wave of them (a
 // workgroup of Hkv waves at 2 waves per SIMD), fewer for small batches.
