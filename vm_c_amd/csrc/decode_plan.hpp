@@ -120,13 +120,28 @@ __device__ __forceinline__ int seq_pages(const DecodeParams& p, int b, int* L_ou
     return L > 0 ? (L + kBs - 1) / kBs : 0;
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const int u = __shfl_up(v, m, 64);
-        if (lane >= m) v += u;
-    }
+// Inclusive prefix sum and non-negative max over the wave in six DPP steps
+// (row_shr 1, 2, 4, 8, then the last lane of the row before, then lane 31): a
+// step is a vector instruction.  Through lane permutes, each step goes by way
+// of the LDS and its latency, and a plan has a dozen of them in a row.
+__device__ __forceinline__ int wave_incl_scan(int v, int) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
     return v;
+}
+__device__ __forceinline__ int plan_wave_sum(int v) { return __builtin_amdgcn_readlane(wave_incl_scan(v, 0), 63); }
+__device__ __forceinline__ int plan_wave_max(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
 // total pages of the batch (one wave, result in every lane)
@@ -135,9 +150,7 @@ __device__ __forceinline__ int total_pages(const DecodeParams& p, int lane) {
     for (int b0 = 0; b0 < p.B; b0 += 64) {
         int L = 0;
         int pg = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) pg += __shfl_xor(pg, m, 64);
-        total += pg;
+        total += plan_wave_sum(pg);
     }
     return total;
 }
@@ -172,17 +185,6 @@ __device__ __forceinline__ int range_of_page(const DecodeParams& p, int64_t g, i
     const int64_t K = ((g + 1) * cn - 1) / T;
     const int64_t w = K < wa * h ? K / wa : h + (K - wa * h) / wb;
     return (int)min(w, (int64_t)n - 1);
-}
-
-__device__ __forceinline__ int plan_wave_sum(int v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-__device__ __forceinline__ int plan_wave_max(int v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = max(v, __shfl_xor(v, m, 64));
-    return v;
 }
 
 // pages and non-empty sequences of the batch (one wave, results in every lane)
@@ -224,8 +226,8 @@ __device__ __forceinline__ void real_pages(const DecodeParams& p, int lane, int 
         const int vs = ps + V * rank, gs = vs - (rank > 0 ? V : 0);
         if (pg > 0 && gs <= v0) best0 = max(best0, v0 < vs ? ps : min(ps + (v0 - vs), ps + pg));
         if (pg > 0 && gs <= v1) best1 = max(best1, v1 < vs ? ps : min(ps + (v1 - vs), ps + pg));
-        carry += __shfl(incl, 63, 64);
-        carry_nz += __shfl(incl_nz, 63, 64);
+        carry += __builtin_amdgcn_readlane(incl, 63);
+        carry_nz += __builtin_amdgcn_readlane(incl_nz, 63);
     }
     *r0 = plan_wave_max(best0);
     *r1 = plan_wave_max(best1);
@@ -270,7 +272,7 @@ __device__ __forceinline__ int collect_segments(const DecodeParams& p, int c_lo,
             }
         }
         ns += __popcll(bal);
-        carry += __shfl(incl, 63, 64);
+        carry += __builtin_amdgcn_readlane(incl, 63);
     }
     return ns;
 }
@@ -303,15 +305,26 @@ __device__ __forceinline__ uint32_t lds16(const uint8_t* p) {
 
 // ------------------------------------------------------------------ merge
 
+// Butterflies over the lanes 32, 16, 8, 4, 2 and 1 apart, without the LDS.
+template <typename F>
+__device__ __forceinline__ float wave_butterfly(float v, F op) {
+    const int lane = threadIdx.x & 63;
+    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
+    swap_pair32(a, b);
+    v = op(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+    a = b = __builtin_bit_cast(uint32_t, v);
+    swap_pair16(a, b);
+    v = op(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+    v = op(v, row_xor<8>(v, lane));
+    v = op(v, row_xor<4>(v, lane));
+    v = op(v, row_xor<2>(v, lane));
+    return op(v, row_xor<1>(v, lane));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-    return v;
+    return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
 }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
+    return wave_butterfly(v, [](float a, float b) { return a + b; });
 }
 
 // Combines the pieces of every sequence that range boundaries cut.  Grid
@@ -323,34 +336,21 @@ __device__ __forceinline__ float wave_sum(float v) {
 __global__ void __launch_bounds__(1024) decode_merge_kernel(DecodeParams p) {
     const int b = blockIdx.x, g = blockIdx.y;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int hq = g * p.G + wave;
-    __shared__ int sh[5];
-    if (wave == 0) {
-        int carry = 0, carry_nz = 0, ps_b = 0, pg_b = 0, rank_b = 0;
-        for (int b0 = 0; b0 < p.B; b0 += 64) {
-            int L = 0;
-            const int pg = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
-            const int nzf = pg > 0 ? 1 : 0;
-            const int incl = wave_incl_scan(pg, lane), incl_nz = wave_incl_scan(nzf, lane);
-            if (b0 + lane == b) {
-                ps_b = carry + incl - pg;
-                pg_b = pg;
-                rank_b = carry_nz + incl_nz - nzf;
-            }
-            carry += __shfl(incl, 63, 64);
-            carry_nz += __shfl(incl_nz, 63, 64);
+    const int hq = g * p.G + __builtin_amdgcn_readfirstlane(wave);
+    int T = 0, nz = 0, ps = 0, pg = 0, rank = 0;
+    for (int b0 = 0; b0 < p.B; b0 += 64) {
+        int L = 0;
+        const int pgl = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
+        const int incl = wave_incl_scan(pgl, lane);
+        const uint64_t some = __ballot(pgl > 0);
+        if (b >= b0 && b < b0 + 64) {  // uniform
+            pg = __builtin_amdgcn_readlane(pgl, b - b0);
+            ps = T + __builtin_amdgcn_readlane(incl, b - b0) - pg;
+            rank = nz + __popcll(some & ((1ull << (b - b0)) - 1));
         }
-        // the lane that held b publishes it
-        if (lane == (b & 63)) {
-            sh[0] = ps_b;
-            sh[1] = pg_b;
-            sh[2] = carry;
-            sh[3] = rank_b;
-            sh[4] = carry_nz;
-        }
+        T += __builtin_amdgcn_readlane(incl, 63);
+        nz += __popcll(some);
     }
-    __syncthreads();
-    const int ps = sh[0], pg = sh[1], T = sh[2], rank = sh[3], nz = sh[4];
     uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + ((int64_t)b * p.Hq + hq) * kD;
     if (pg == 0) {
         reinterpret_cast<uint32_t*>(orow)[lane] = 0u;
@@ -455,10 +455,10 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
         const int pg = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
         const int incl = wave_incl_scan(pg, lane);
         if (b >= b0 && b < b0 + 64) {  // uniform over the wave
-            ps_b = __shfl(carry + incl - pg, b - b0, 64);
-            pg_b = __shfl(pg, b - b0, 64);
+            pg_b = __builtin_amdgcn_readlane(pg, b - b0);
+            ps_b = carry + __builtin_amdgcn_readlane(incl, b - b0) - pg_b;
         }
-        carry += __shfl(incl, 63, 64);
+        carry += __builtin_amdgcn_readlane(incl, 63);
     }
     const int T = carry;
     uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + ((int64_t)b * p.Hq + hq) * D + NV * lane;
