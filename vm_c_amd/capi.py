@@ -7,6 +7,8 @@ if the library is missing or a call fails, this raises.
 import ctypes as C
 import os
 
+import torch
+
 PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG, "libvmc_attn.so")
 
@@ -117,18 +119,21 @@ def _check(rc, what):
         raise VmcError(f"{what} failed with status {rc}")
 
 
+# A decode step is two calls of a few microseconds of GPU time each, so what a
+# call costs here counts: addresses go to ctypes as plain integers (the
+# argtypes make them pointers), and the current stream's handle is asked for
+# without a torch.cuda.Stream object around it.
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(stream=None):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dtype_code(t):
-    import torch
     if t.dtype == torch.float16:
         return DTYPE_F16
     if t.dtype == torch.bfloat16:
