@@ -393,10 +393,10 @@ int vmc_flash_attention_prefill(void* output, const void* query, const void* key
  * workspace / workspace_bytes, at least
  * vmc_flash_attention_prefill_workspace_size(num_tokens, num_kv_heads,
  * head_dim) bytes, 16-byte aligned (VMC_ENOMEM when smaller, VMC_EINVAL when
- * NULL at head_dim 128).  A first launch writes the fp16 V^T tiles of the
- * step's V (16 KB per 64 keys and KV head) into the workspace once, so the
- * attention kernel fetches them instead of transposing V in every
- * workgroup that reads it.  Outputs equal vmc_flash_attention_prefill's bit
+ * NULL at head_dim 128).  In bf16 a first launch writes the fp16 V^T tiles of
+ * the step's V (16 KB per 64 keys and KV head) into the workspace once, so the
+ * attention kernel fetches them instead of transposing V in every workgroup
+ * that reads it; fp16 steps do not use it.  Outputs equal vmc_flash_attention_prefill's bit
  * for bit, except that bf16 V which that function would run in its exact
  * mode for some workgroups may run exact in more of them here (a tile's
  * flag covers all of its rows).  head_dim 64 / 256 ignore the workspace.

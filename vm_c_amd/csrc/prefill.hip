@@ -19,10 +19,9 @@ namespace {
 // the byte image of prefill_kernel's LDS V^T tile: fp16 V[64 tau + 16c + 8a
 // + 4h + e][d] at byte d * 128 + 16 * ((2c + h) ^ ((d >> 1) & 7)) + 8a + 2e
 // (keys past the step: zero).  flag[g][tau] = 1 when some row of the tile
-// holds, for bf16 V, |v| >= 65536 or a NaN, or a value below 2^-17 and none
-// of 2^-8 or more (per row: every case the kernel's own pass flags for its
-// rows' groups is flagged); for fp16 V, an inf or NaN.
-template <bool BF16>
+// holds |v| >= 65536 or a NaN, or a value below 2^-17 and none of 2^-8 or more
+// (per row: every case the kernel's own pass flags for its rows' groups is
+// flagged).
 __global__ void __launch_bounds__(256) vt_prep_kernel(const uint16_t* __restrict__ v, uint8_t* __restrict__ vt,
                                                       uint8_t* __restrict__ flag, int T, int Hkv, int ntT) {
     // rows padded to 65 dwords: the 8 lanes that gather one dim from 8 rows
@@ -44,11 +43,9 @@ __global__ void __launch_bounds__(256) vt_prep_kernel(const uint16_t* __restrict
             const u16x2 a = __builtin_bit_cast(u16x2, w[e] & 0x7fff7fffu);
             amax = __builtin_elementwise_max(amax, a);
             amin1 = __builtin_elementwise_min(amin1, a - u16x2{1, 1});
-            if constexpr (BF16) {
-                const f16x2 hh = {(_Float16)__builtin_bit_cast(float, w[e] << 16),
-                                  (_Float16)__builtin_bit_cast(float, w[e] & 0xffff0000u)};
-                w[e] = __builtin_bit_cast(uint32_t, hh);
-            }
+            const f16x2 hh = {(_Float16)__builtin_bit_cast(float, w[e] << 16),
+                              (_Float16)__builtin_bit_cast(float, w[e] & 0xffff0000u)};
+            w[e] = __builtin_bit_cast(uint32_t, hh);
         }
         mx = max((uint32_t)amax[0], (uint32_t)amax[1]);
         mn1 = min((uint32_t)amin1[0], (uint32_t)amin1[1]);
@@ -59,11 +56,8 @@ __global__ void __launch_bounds__(256) vt_prep_kernel(const uint16_t* __restrict
             mn1 = min(mn1, (uint32_t)__shfl_xor((int)mn1, m, kWave));
         }
         // bf16 bit patterns: 0x477f = 65280 (largest below 2^16), 0x3700 =
-        // 2^-17, 0x3b80 = 2^-8; fp16: 0x7c00 = inf
-        if constexpr (BF16)
-            fl |= mx > 0x477fu || (mn1 < 0x36ffu && mx < 0x3b80u);
-        else
-            fl |= mx >= 0x7c00u;
+        // 2^-17, 0x3b80 = 2^-8
+        fl |= mx > 0x477fu || (mn1 < 0x36ffu && mx < 0x3b80u);
 #pragma unroll
         for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(&tl[r][8 * cc + 2 * e]) = w[e];
     }
@@ -262,8 +256,13 @@ extern "C" int vmc_flash_attention_prefill_v2(void* output, const void* query, c
 }
 
 namespace {
-// the local prefill; with a workspace (ws != NULL) the V^T tiles are built
-// once by vt_prep_kernel and the attention kernel fetches them
+// the local prefill; with a workspace (ws != NULL) the V^T tiles of a bf16 step
+// are built once by vt_prep_kernel and the attention kernel fetches them.  In
+// fp16 a workgroup's own transpose needs no conversion and no range check and
+// costs less than the extra launch saves, 32/8 heads, us prebuilt / own: 64
+// tokens 13.8 / 9.6, 512 tokens 20.9 / 18.1, 1024 tokens 31.3 / 28.1, 4096
+// tokens 157 / 154, 2 x 4096 tokens 301 / 297 (64/8 heads 571 / 576; bf16, 2 x
+// 4096 tokens: 296 / 319)
 int local_prefill(void* output, const void* query, const void* key, const void* value, int num_tokens,
                   int num_heads, int num_kv_heads, int head_dim, float scale, const int32_t* token_positions,
                   int dtype, void* key_cache, void* value_cache, const int64_t* slot_mapping, int64_t block_size,
@@ -333,9 +332,11 @@ int local_prefill(void* output, const void* query, const void* key, const void* 
     if ((int64_t)prm.ntiles * prm.Hkv * prm.hgroups > 0x7fffffffLL) return VMC_EINVAL;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const bool bf = dtype == VMC_DTYPE_BF16;
-    if (!ws) return launch_tiled(prm, bf, fmt, SRC_LOCAL, false, s);
-    if (ws_bytes < vt_workspace_bytes(num_tokens, num_kv_heads)) return VMC_ENOMEM;
-    if (((uintptr_t)ws & 15) != 0) return VMC_EINVAL;
+    if (ws) {
+        if (ws_bytes < vt_workspace_bytes(num_tokens, num_kv_heads)) return VMC_ENOMEM;
+        if (((uintptr_t)ws & 15) != 0) return VMC_EINVAL;
+    }
+    if (!ws || !bf) return launch_tiled(prm, bf, fmt, SRC_LOCAL, false, s);
     const int ntT = (num_tokens + BN - 1) / BN;
     prm.vt = reinterpret_cast<const uint8_t*>(ws);
     prm.vt_flag = prm.vt + (int64_t)ntT * num_kv_heads * (kD * BN * 2);
@@ -343,13 +344,9 @@ int local_prefill(void* output, const void* query, const void* key, const void* 
     uint8_t* vt = reinterpret_cast<uint8_t*>(ws);
     uint8_t* flag = vt + (int64_t)ntT * num_kv_heads * (kD * BN * 2);
     const dim3 vgrid((unsigned)ntT, (unsigned)num_kv_heads);
-    if (bf)
-        hipLaunchKernelGGL(vt_prep_kernel<true>, vgrid, dim3(256), 0, s, prm.v, vt, flag, num_tokens, num_kv_heads, ntT);
-    else
-        hipLaunchKernelGGL(vt_prep_kernel<false>, vgrid, dim3(256), 0, s, prm.v, vt, flag, num_tokens, num_kv_heads,
-                           ntT);
+    hipLaunchKernelGGL(vt_prep_kernel, vgrid, dim3(256), 0, s, prm.v, vt, flag, num_tokens, num_kv_heads, ntT);
     VMC_LAUNCH_CHECK();
-    return launch_tiled(prm, bf, fmt, SRC_LOCAL, true, s);
+    return launch_tiled(prm, true, fmt, SRC_LOCAL, true, s);
 }
 }  // namespace
 

@@ -100,7 +100,7 @@ struct PrefillParams {
 // The kernel of (bf16, fmt, src, vt), one translation unit per key split:
 // KS = 1, a wave takes a tile's 64 keys; KS = 2, the halves of a tile go to
 // two waves (prefill_split.hip).  fmt: the fused append's format or -1; src:
-// SRC_*; vt: prebuilt V^T tiles (local K/V).
+// SRC_*; vt: prebuilt V^T tiles (local bf16 K/V).
 int launch_prefill_whole(PrefillParams& prm, bool bf16, int fmt, int src, bool vt, hipStream_t s);
 int launch_prefill_split(PrefillParams& prm, bool bf16, int fmt, int src, bool vt, hipStream_t s);
 
@@ -971,16 +971,9 @@ prefill_kernel(PrefillParams p) {
                 const uint8_t* fl = p.vt_flag + (int64_t)g * p.vt_tiles + kv_lo / BN;
                 for (int t0 = 0; t0 < ntile; t0 += 64)
                     flagged |= __ballot(t0 + lane < ntile && fl[t0 + lane] != 0) != 0;
-                // a flagged tile: bf16 runs the exact mode; fp16 (whose flag
-                // marks an inf or NaN, possibly in another sequence's rows of
-                // the tile) transposes its own rows, which stop at kv_end
-                if (!flagged) {
-                    run(std::false_type{}, std::true_type{});
-                    prebuilt = true;
-                } else if constexpr (BF16) {
-                    run(std::true_type{}, std::false_type{});
-                    prebuilt = true;
-                }
+                if (flagged) run(std::true_type{}, std::false_type{});  // the exact mode
+                else run(std::false_type{}, std::true_type{});
+                prebuilt = true;
             }
         }
         if (!prebuilt) run_pass();
@@ -1130,8 +1123,7 @@ template <int KS>
 int launch_prefill_any(PrefillParams& prm, bool bf16, int fmt, int src, bool vt, hipStream_t s) {
     switch (src) {
         case SRC_LOCAL:
-            if (vt) return bf16 ? launch_prefill_local<true, true, KS>(prm, fmt, s)
-                                : launch_prefill_local<false, true, KS>(prm, fmt, s);
+            if (vt) return bf16 ? launch_prefill_local<true, true, KS>(prm, fmt, s) : VMC_EINVAL;
             return bf16 ? launch_prefill_local<true, false, KS>(prm, fmt, s)
                         : launch_prefill_local<false, false, KS>(prm, fmt, s);
         case SRC_PAGED:
