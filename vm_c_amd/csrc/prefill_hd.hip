@@ -6,8 +6,8 @@
 // What bounds it: the matrix cores (4 D flops per query, key and head; P V
 // counts two or three times, see below).  The one-wave-per-row kernel had no
 // products and read K/V once per row (22.9 ms for 10,752 tokens in 4 prompts,
-// 16/2 heads, head_dim 256, bf16: 12.5 TFLOP/s); this one takes 560 us (510
-// TFLOP/s of the attention's own flops, 1.02 PFLOP/s on the matrix cores).
+// 16/2 heads, head_dim 256, bf16: 12.5 TFLOP/s); this one takes 535 us (533
+// TFLOP/s of the attention's own flops, 1.07 PFLOP/s on the matrix cores).
 // Workgroup = 8 waves = up to 4 query heads of one KV head x 32-row query
 // blocks, as prefill_kernel (prefill.hip), so a K/V tile of 64 keys in LDS
 // serves 256 query rows.  Tiles arrive by load-to-LDS transfers: three slots
@@ -233,13 +233,27 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
             for (int b = 0; b < HB; ++b)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) sacc[b][i] = 0.0f;
-#pragma unroll
-            for (int s = 0; s < D / 16; ++s)
+            // K operands are read two steps ahead of their products, V operands
+            // one.  Fixed by scheduling barriers: left alone, the compiler
+            // issues each read right before the product that waits for it (593
+            // against 565 us on the 4 prompts named above, with the store).
+            u32x4 ka[3][HB];
+            auto read_k = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
                 for (int b = 0; b < HB; ++b)
-                    sacc[b] = M::mma(as_v8<V8>(lds128((k_slot ^ (uint32_t)(32 * (s & 7))) +
-                                                      (uint32_t)((HB * r + b) * 32 * ROW + 256 * (s >> 3)))),
-                                     qf[s], sacc[b]);
+                    ka[s % 3][b] = lds128((k_slot ^ (uint32_t)(32 * (s & 7))) +
+                                          (uint32_t)((HB * r + b) * 32 * ROW + 256 * (s >> 3)));
+            };
+            read_k(0);
+            read_k(1);
+#pragma unroll
+            for (int s = 0; s < D / 16; ++s) {
+                if (s + 2 < D / 16) read_k(s + 2);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < HB; ++b) sacc[b] = M::mma(as_v8<V8>(ka[s % 3][b]), qf[s], sacc[b]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if (need_mask) {
 #pragma unroll
                 for (int b = 0; b < HB; ++b)
@@ -286,17 +300,26 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
                     }
                 }
             l_part += sum;
+            // O^T += V^T P^T, V operands (two transposing reads each) one ahead
+            u32x2 va[2][2];
+            auto read_v = [&](int i) __attribute__((always_inline)) {
+                const int c = i / (D / 32), m = i % (D / 32);
+                const int vo = (2 * HB * r + c) * 16 * ROW + 256 * (m >> 2);
 #pragma unroll
-            for (int c = 0; c < 2 * HB; ++c) {
+                for (int sec = 0; sec < 2; ++sec)
+                    va[i & 1][sec] = lds_tr((v_slot[sec] ^ (uint32_t)(64 * (m & 3))) + (uint32_t)vo);
+            };
+            constexpr int NV = 2 * HB * (D / 32);
+            read_v(0);
 #pragma unroll
-                for (int m = 0; m < D / 32; ++m) {
-                    const int vo = (2 * HB * r + c) * 16 * ROW + 256 * (m >> 2);
-                    const u32x2 a0 = lds_tr((v_slot[0] ^ (uint32_t)(64 * (m & 3))) + (uint32_t)vo);
-                    const u32x2 a1 = lds_tr((v_slot[1] ^ (uint32_t)(64 * (m & 3))) + (uint32_t)vo);
-                    const V8 va = as_v8<V8>(u32x4{a0[0], a0[1], a1[0], a1[1]});
+            for (int i = 0; i < NV; ++i) {
+                if (i + 1 < NV) read_v(i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                const int c = i / (D / 32), m = i % (D / 32);
+                const V8 x = as_v8<V8>(u32x4{va[i & 1][0][0], va[i & 1][0][1], va[i & 1][1][0], va[i & 1][1][1]});
 #pragma unroll
-                    for (int u = 0; u < NTERM; ++u) o[m] = M::mma(va, as_v8<V8>(pt[u][c]), o[m]);
-                }
+                for (int u = 0; u < NTERM; ++u) o[m] = M::mma(x, as_v8<V8>(pt[u][c]), o[m]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
