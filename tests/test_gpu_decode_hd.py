@@ -113,11 +113,14 @@ def test_prefill_rows(dev, d, splits):
 
 
 # infinities and NaNs: V of a key whose weight is 0, V of one that counts, K,
-# q; scores far enough apart that weights underflow
+# q; scores far enough apart that weights underflow.  Whole sequences, and ones
+# cut into as many or at most 3 pieces a row: there a piece that met one is
+# computed key by key and merged with the others' products
 @pytest.mark.parametrize("d", [64, 256])
 @pytest.mark.parametrize("fmt,qt", [(F16, "f16"), (BF16, "bf16"), (Q8, "f16")])
+@pytest.mark.parametrize("splits", [0, 1, 3])
 @pytest.mark.parametrize("what", ["v_unused", "v_inf", "k_nan", "k_inf", "q_nan", "spread"])
-def test_decode_specials(dev, d, fmt, qt, what):
+def test_decode_specials(dev, d, fmt, qt, splits, what):
     from vm_c_amd import capi
 
     def edit(w, K, V, Q):
@@ -137,6 +140,7 @@ def test_decode_specials(dev, d, fmt, qt, what):
             Q.mul_(8.0)
 
     w, Q, pages, lens, Hkv, scale, kw = _setup(dev, d, (4, 2), fmt, qt, False, seed=13, edit=edit)
-    got, ref, ulp = _both(Q, lambda o: capi.paged_attention_decode(o, Q, *pages, lens, Hkv, scale, max_splits=1, **kw))
+    got, ref, ulp = _both(Q, lambda o: capi.paged_attention_decode(o, Q, *pages, lens, Hkv, scale, max_splits=splits,
+                                                                   **kw))
     # scores of order 100: their fp32 sums differ by up to 2^-24 * 2^7 * a few, and so do the weights, relatively
     _close(got, ref, ulp, atol=2e-4 if what == "spread" else 2e-5)

@@ -438,7 +438,9 @@ __global__ void __launch_bounds__(1024) decode_merge_kernel(DecodeParams p) {
     *reinterpret_cast<u32x4*>(orow + 8 * r16) = u32x4{w4[0], w4[1], w4[2], w4[3]};
 }
 
-// The same combination over rows of D + 4 floats, four waves per (sequence,
+// The same combination over rows of D + 4 floats (o, m, l: o and l are sums of
+// weights 2^(s - m), s the score in log2 units, whichever loop wrote the row;
+// no key: m = -inf, l = 0), four waves per (sequence,
 // query head): grid (B, Hq), 256 threads; wave w takes pieces w, w + 4, ...
 // (sixteen rows in flight, so 64 pieces cost one round of loads), lane l dims
 // l D / 64 .. ; the four partial sums meet in LDS.

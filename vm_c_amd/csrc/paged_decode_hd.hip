@@ -410,7 +410,8 @@ __global__ void __launch_bounds__((D == 64 ? 256 : 128), (D == 64 ? 3 : 2)) page
                 float* pp = p.part + (slot * p.Hq + (int64_t)g * p.G + r16) * (D + 4);
 #pragma unroll
                 for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(pp + 16 * t + 4 * grp) = o[t];
-                if (grp == 0) *reinterpret_cast<float2*>(pp + D) = make_float2(m_run, l);
+                // o and l hold weights of 2^(s - m_run + kOff): the reference they go with
+                if (grp == 0) *reinterpret_cast<float2*>(pp + D) = make_float2(m_run - kOff, l);
             }
         }
         if (badb) {
