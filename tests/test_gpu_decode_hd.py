@@ -52,7 +52,7 @@ def _both(Q, run):
 
 def _close(got, ref, ulp, atol=2e-5):
     import torch
-    bad = (got - ref).abs() > atol + ulp * ref.abs()
+    bad = ~((got - ref).abs() <= atol + ulp * ref.abs())  # a NaN or an infinity on one side is bad too
     bad &= ~((got == ref) | (got.isnan() & ref.isnan()))
     assert not bad.any(), f"{int(bad.sum())} values differ, first at {torch.nonzero(bad)[0].tolist()}: " \
                           f"{got[bad][0].item()} vs {ref[bad][0].item()}"
@@ -112,14 +112,15 @@ def test_prefill_rows(dev, d, splits):
     _close(got, ref, ulp)
 
 
-# infinities and NaNs: V of a key whose weight is 0, V of one that counts, K,
-# q; scores far enough apart that weights underflow.  Whole sequences, and ones
+# infinities and NaNs: V of a key whose weight is 0 (alone, and among 20 pages
+# of such keys, so that whole pieces are), V of one that counts (the last one
+# too), K, q; scores far enough apart that weights underflow.  Whole sequences, and ones
 # cut into as many or at most 3 pieces a row: there a piece that met one is
 # computed key by key and merged with the others' products
 @pytest.mark.parametrize("d", [64, 256])
 @pytest.mark.parametrize("fmt,qt", [(F16, "f16"), (BF16, "bf16"), (Q8, "f16")])
 @pytest.mark.parametrize("splits", [0, 1, 3])
-@pytest.mark.parametrize("what", ["v_unused", "v_inf", "k_nan", "k_inf", "q_nan", "spread"])
+@pytest.mark.parametrize("what", ["v_unused", "v_far", "v_inf", "v_last", "k_nan", "k_inf", "q_nan", "spread"])
 def test_decode_specials(dev, d, fmt, qt, splits, what):
     from vm_c_amd import capi
 
@@ -128,6 +129,11 @@ def test_decode_specials(dev, d, fmt, qt, splits, what):
         if what == "v_unused":
             K[row, 0, :] = -30 * Q[6, 0, :].sign()
             V[row, 0, 3] = float("inf")
+        elif what == "v_far":
+            K[row + 280:row + 600, 0, :] = -30 * Q[6, 0, :].sign()
+            V[row + 400, 0, 3] = float("inf")
+        elif what == "v_last":
+            V[row - 40 + 1499, 0, 3] = float("inf")
         elif what == "v_inf":
             V[row, 0, 3] = float("inf")
         elif what == "k_nan":

@@ -440,7 +440,9 @@ __global__ void __launch_bounds__(1024) decode_merge_kernel(DecodeParams p) {
 
 // The same combination over rows of D + 4 floats (o, m, l: o and l are sums of
 // weights 2^(s - m), s the score in log2 units, whichever loop wrote the row;
-// no key: m = -inf, l = 0), four waves per (sequence,
+// no key: m = -inf, l = 0).  A piece of weight 0 adds nothing, also where its o
+// holds an infinity: the key that brought it has weight 0 in the whole row (an
+// l that is NaN, from a score that is, stays one).  Four waves per (sequence,
 // query head): grid (B, Hq), 256 threads; wave w takes pieces w, w + 4, ...
 // (sixteen rows in flight, so 64 pieces cost one round of loads), lane l dims
 // l D / 64 .. ; the four partial sums meet in LDS.
@@ -504,18 +506,20 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
         for (int u = 0; u < 16; ++u) mx = s0 + 4 * u < nseg ? fmaxf(mx, ml[u].x) : mx;
         if (mx > M && M != kNegInf) {  // wave-uniform
             const float f = __builtin_amdgcn_exp2f(M - mx);
+            const bool none = f == 0.0f && L == L;
             L *= f;
 #pragma unroll
-            for (int e = 0; e < NV; ++e) acc[e] *= f;
+            for (int e = 0; e < NV; ++e) acc[e] = none ? 0.0f : acc[e] * f;
         }
         M = mx;
         const float Mu = M == kNegInf ? 0.0f : M;
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
             const float wu = s0 + 4 * u < nseg ? __builtin_amdgcn_exp2f(ml[u].x - Mu) : 0.0f;
+            const bool none = wu == 0.0f && ml[u].y == ml[u].y;
             L = __builtin_fmaf(ml[u].y, wu, L);
 #pragma unroll
-            for (int e = 0; e < NV; ++e) acc[e] = __builtin_fmaf(o[u][e], wu, acc[e]);
+            for (int e = 0; e < NV; ++e) acc[e] = __builtin_fmaf(none ? 0.0f : o[u][e], wu, acc[e]);
         }
     }
     *reinterpret_cast<fv*>(&red[wave][NV * lane]) = acc;
@@ -534,10 +538,11 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const float f = red[w][D] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(red[w][D] - Mgu);
+        const bool none = f == 0.0f && red[w][D + 1] == red[w][D + 1];
         Lg = __builtin_fmaf(red[w][D + 1], f, Lg);
         const fv v = *reinterpret_cast<const fv*>(&red[w][NV * lane]);
 #pragma unroll
-        for (int e = 0; e < NV; ++e) og[e] = __builtin_fmaf(v[e], f, og[e]);
+        for (int e = 0; e < NV; ++e) og[e] = __builtin_fmaf(none ? 0.0f : v[e], f, og[e]);
     }
     const float inv = Lg > 0.0f ? 1.0f / Lg : 0.0f;
 #pragma unroll
