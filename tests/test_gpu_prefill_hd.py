@@ -60,14 +60,20 @@ def test_prefill_any_positions(dev, d):
 
 
 # infinities and NaNs in q, K and V (a row sees only its own window's), values
-# near the largest of the type, scores far apart
+# near the largest of the type (v_late: the sums stay below it only with weights
+# of at most 1, and the scores rise by 5 after the first tile, less than moves
+# the kernel's reference max), scores far apart
 @pytest.mark.parametrize("d", [64, 256])
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("what", ["v_inf", "k_nan", "q_inf", "v_large", "spread"])
+@pytest.mark.parametrize("what", ["v_inf", "k_nan", "q_inf", "v_large", "v_late", "spread"])
 def test_prefill_specials(dev, d, bf16, what):
     from vm_c_amd import capi
     q, k, v, pos, _ = _inputs(dev, d, (4, 2), [90, 150], bf16, seed=6)
     big = 1e30 if bf16 else 60000.0
+    if what == "v_late":
+        big = 2.0 ** 121 if bf16 else 60000.0
+        v.copy_(big / 8 * v.abs().clamp_(0.5, 8))
+        q[:, :, 0], k[:, :, 0], k[90 + 64:, :, 0] = d ** 0.5, 0, 5
     if what == "v_inf":
         v[100, 0, 3] = float("inf")
     elif what == "k_nan":
@@ -76,8 +82,10 @@ def test_prefill_specials(dev, d, bf16, what):
         q[95, 2, 1] = float("inf")
     elif what == "v_large":
         v.mul_(big / 8).clamp_(-big, big)
-    else:
+    elif what == "spread":
         q.mul_(8.0)
     got, ref, ulp = _both(q, lambda o: capi.flash_attention_prefill(o, q, k, v, pos, 2, 1 / np.sqrt(d)))
     # scores of order 100: their fp32 sums differ by up to 2^-24 * 2^7 * a few, and so do the weights, relatively
-    _close(got, ref, ulp, atol=2e-5 * big / 8 if what == "v_large" else 2e-4 if what == "spread" else 2e-5)
+    if what == "v_late":
+        assert ref.isfinite().all()
+    _close(got, ref, ulp, atol=2e-5 * big / 8 if what in ("v_large", "v_late") else 2e-4 if what == "spread" else 2e-5)

@@ -28,8 +28,9 @@
 // 590 us on the case above with its append, the same error against 64 bits in
 // the bf16 output (1.6e-3) but five times the wrongly rounded values (2.4e-3
 // of them against 4.4e-4; three terms 3.1e-4).  V of either type enters
-// exactly.  A row whose products met an infinity or a NaN reruns key
-// by key (gen_row).
+// exactly.  A row whose sums are not finite reruns key by key (gen_row): its
+// products met an infinity or a NaN, or bf16 V so large that weights of up to
+// 2^8 (the reference max lags by that much) overflow where weights of 1 do not.
 #include "generic_row.hpp"
 #include "prefill_dev.hpp"
 #include "prefill_hd.hpp"
@@ -348,7 +349,7 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
 #pragma unroll
     for (int m = 0; m < D / 32; ++m)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) bad |= !(o[m][i] == o[m][i]);
+        for (int i = 0; i < 16; ++i) bad |= !(fabsf(o[m][i]) < __builtin_inff());
     uint64_t badb = __ballot(bad && row_ok);
     badb = (badb | (badb >> 32)) & 0xffffffffull;  // a row is the lane and its partner
     if (row_ok && !((badb >> c32) & 1)) {
