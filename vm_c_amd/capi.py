@@ -147,7 +147,8 @@ SELFTEST_CHECKS = {1: "sum over rows", 2: "max over rows", 4: "LDS gather",
                    256: "mfma 16x16x16 f16 subnormal operands", 512: "LDS gather from the diagonal",
                    1024: "mfma 16x16x32 f16 subnormal operands",
                    2048: "bf16 conversion instruction vs the integer rounding rule",
-                   4096: "16-lane DPP xor exchanges", 8192: "16-lane DPP row sum"}
+                   4096: "16-lane DPP xor exchanges", 8192: "16-lane DPP row sum",
+                   16384: "16-bit terms of a weight"}
 
 
 def selftest():

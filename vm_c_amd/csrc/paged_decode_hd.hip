@@ -24,14 +24,15 @@
 // K reads (f is a bijection on the rows that share banks) and for the
 // transposing reads of 8 rows x 32 bytes.
 //
-// Weights stay fp32-exact: P enters the products as a sum of 16-bit terms,
-// two fp16 terms (22 bits; scaled by 2^15, so that a weight of 2^-39 is still
-// there) against fp16 V, three bf16 terms (24 bits) otherwise.  q8_0 / q4_0
+// Weights keep their 24 bits: P enters the products as a sum of three 16-bit
+// terms (weight_terms.hpp), fp16 against fp16 V (the largest weight scaled to
+// 2^15: whole down to 2^-16, off by at most 2^-40 below), bf16 otherwise.  q8_0 / q4_0
 // codes are integers of at most 8 bits, exact in either type; a block's scale
 // multiplies its partial score (K) or the weights (V) in fp32.
 #include "decode_plan.hpp"
 #include "generic_row.hpp"
 #include "paged_decode_hd.hpp"
+#include "weight_terms.hpp"
 
 namespace vmc {
 namespace {
@@ -61,14 +62,6 @@ struct HdT<true> {
 template <bool BF>
 __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
     return (uint32_t)f32_to_half<BF>(a) | ((uint32_t)f32_to_half<BF>(b) << 16);
-}
-// packed 16-bit rounding of (a, b); a and b become what it left out
-template <bool BF>
-__device__ __forceinline__ uint32_t split_term(float& a, float& b) {
-    const uint32_t w = pack_half2<BF>(a, b);
-    a -= half_to_f32<BF>((uint16_t)(w & 0xffffu));
-    b -= half_to_f32<BF>((uint16_t)(w >> 16));
-    return w;
 }
 
 template <int D, int FMT>
@@ -133,7 +126,7 @@ __global__ void __launch_bounds__((D == 64 ? 256 : 128), (D == 64 ? 3 : 2)) page
     constexpr int PG = GE::pg, TOK = GE::tok, NT = D / 16, NP = 4 * PG;
     constexpr bool kGguf = GE::gguf;
     constexpr bool VBF = kGguf || FMT == FMT_BF16;  // type of the V operand and the weights' terms
-    constexpr int kTerms = VBF ? 3 : 2;
+    constexpr int kTerms = WeightTerms<VBF>::n;
     constexpr float kOff = VBF ? 0.0f : 15.0f;  // weights are 2^(s - m + kOff)
     struct WaveLds {
         uint8_t k[GE::tile], v[GE::tile];
@@ -306,9 +299,12 @@ __global__ void __launch_bounds__((D == 64 ? 256 : 128), (D == 64 ? 3 : 2)) page
         uint32_t pt[kTerms][NP / 2];
         auto split = [&](float (&x)[NP]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < kTerms; ++u)
+            for (int i = 0; i < NP; i += 2) {
+                uint32_t w[kTerms];
+                WeightTerms<VBF>::split(x[i], x[i + 1], w);
 #pragma unroll
-                for (int i = 0; i < NP; i += 2) pt[u][i / 2] = split_term<VBF>(x[i], x[i + 1]);
+                for (int u = 0; u < kTerms; ++u) pt[u][i / 2] = w[u];
+            }
         };
         if constexpr (!kGguf) split(pr);
 #pragma unroll

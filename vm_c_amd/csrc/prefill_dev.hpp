@@ -16,7 +16,6 @@ struct MT<true> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ uint16_t cvt(float x) { return f32_to_bf16_bits(x); }
-    static __device__ __forceinline__ float back(uint16_t b) { return bf16_bits_to_f32(b); }
 };
 template <>
 struct MT<false> {
@@ -25,7 +24,6 @@ struct MT<false> {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ uint16_t cvt(float x) { return f32_to_f16_bits(x); }
-    static __device__ __forceinline__ float back(uint16_t b) { return f16_bits_to_f32(b); }
 };
 
 template <typename V8>

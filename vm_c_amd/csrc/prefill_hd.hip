@@ -4,7 +4,7 @@
 // which keeps operands that are not 16-byte aligned.
 //
 // What bounds it: the matrix cores (4 D flops per query, key and head; P V
-// counts two or three times, see below).  The one-wave-per-row kernel had no
+// counts three times, see below).  The one-wave-per-row kernel had no
 // products and read K/V once per row (22.9 ms for 10,752 tokens in 4 prompts,
 // 16/2 heads, head_dim 256, bf16: 12.5 TFLOP/s); this one takes 535 us (533
 // TFLOP/s of the attention's own flops, 1.07 PFLOP/s on the matrix cores).
@@ -18,22 +18,27 @@
 //   32 lanes on).  V^T operands come from the row-major tile by transposing
 //   LDS reads; the contraction index is permuted as P leaves the S registers
 //   (k = 8h + e <-> key 16c + 8 (e / 4) + 4h + e % 4).  Their LDS time hides
-//   under the products, which take two or three MFMAs for each operand read.
+//   under the products, which take three MFMAs for each operand read.
 // Head_dim 256 runs the softmax per 32 keys and 64 per 64: O, Q and S then
 // fit the 256 registers of a wave at two waves per SIMD.
 //
-// Weights keep their fp32 precision: P is the sum of rounded 16-bit terms of
-// V's own type, an MFMA each: two fp16 terms (22 bits; scaled by 2^7 against
-// underflow), three bf16 terms (24 bits).  Two bf16 terms took 475 instead of
-// 590 us on the case above with its append, the same error against 64 bits in
-// the bf16 output (1.6e-3) but five times the wrongly rounded values (2.4e-3
-// of them against 4.4e-4; three terms 3.1e-4).  V of either type enters
+// Weights keep their 24 bits: P is the sum of three rounded 16-bit terms of V's
+// own type, an MFMA each (weight_terms.hpp; fp16: scaled by 2^7 against
+// underflow).  Two bf16 terms took 475 instead of 590 us on the case above with
+// its append, the same error against 64 bits in the bf16 output (1.6e-3) but
+// five times the wrongly rounded values (2.4e-3 of them against 4.4e-4; three
+// terms 3.1e-4).  Two fp16 terms took 166 instead of 204 us (head_dim 64, 32/8
+// heads, 4096 tokens) and 261 instead of 330 us (256, 16/2); they leave 22 bits
+// of a weight, which no N(0, 1) input showed in the fp16 output (both round
+// 1.8e-3 of the values wrongly at 256, the one-wave kernel 3.8e-3).  V of either
+// type enters
 // exactly.  A row whose sums are not finite reruns key by key (gen_row): its
 // products met an infinity or a NaN, or bf16 V so large that weights of up to
 // 2^8 (the reference max lags by that much) overflow where weights of 1 do not.
 #include "generic_row.hpp"
 #include "prefill_dev.hpp"
 #include "prefill_hd.hpp"
+#include "weight_terms.hpp"
 
 namespace vmc {
 namespace {
@@ -106,7 +111,7 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
     constexpr int NS = D == 256 ? 2 : 3;        // tile slots
     constexpr int ROW = 2 * D, TILE = kHdBN * ROW;
     constexpr int NTR = TILE / (1024 * kHdW);   // transfers per wave and tensor
-    constexpr int NTERM = BF ? 3 : 2;           // 16-bit terms of a weight
+    constexpr int NTERM = WeightTerms<BF>::n;   // 16-bit terms of a weight
     constexpr int HB = D == 256 ? 1 : 2;        // 32-key blocks per softmax round
     constexpr float kOff = BF ? 0.0f : 7.0f;    // weights are 2^(s - m + kOff), at most 2^15
     struct Lds {
@@ -292,13 +297,10 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
                     float x0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[c >> 1][j], csc, -ref));
                     float x1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[c >> 1][j + 1], csc, -ref));
                     sum += x0 + x1;
+                    uint32_t x[NTERM];
+                    WeightTerms<BF>::split(x0, x1, x);
 #pragma unroll
-                    for (int u = 0; u < NTERM; ++u) {
-                        const uint32_t x = (uint32_t)M::cvt(x0) | ((uint32_t)M::cvt(x1) << 16);
-                        x0 -= M::back((uint16_t)(x & 0xffffu));
-                        x1 -= M::back((uint16_t)(x >> 16));
-                        pt[u][c][e >> 1] = x;
-                    }
+                    for (int u = 0; u < NTERM; ++u) pt[u][c][e >> 1] = x[u];
                 }
             l_part += sum;
             // O^T += V^T P^T, V operands (two transposing reads each) one ahead

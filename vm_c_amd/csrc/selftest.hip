@@ -2,10 +2,12 @@
 // on: cross-row reductions, the wave-private LDS gathers, the operand /
 // result layouts of the MFMA shapes used (16x16x32 f16/bf16, 16x16x16 f16,
 // 32x32x16 f16/bf16), exact fp16 subnormal operands in the 16x16x16 MFMA,
-// the bf16 conversion instruction and the 16-lane DPP exchanges.  One wave,
+// the bf16 conversion instruction, the 16-lane DPP exchanges and what the
+// 16-bit terms of a weight leave out.  One wave,
 // fixed inputs (small integers where arithmetic is checked), every lane
 // compares its own results with the expected values.
 #include "vmc_common.hpp"
+#include "weight_terms.hpp"
 
 namespace vmc {
 namespace {
@@ -14,7 +16,7 @@ enum {
     kSumGroups = 1, kMaxGroups = 2, kGather = 4, kMfma16x32 = 8, kMfma16x16 = 16,
     kMfma32x16 = 32, kMfma16x32bf = 64, kMfma32x16bf = 128, kMfma16x16Subnormal = 256,
     kGatherDiag = 512, kMfma16x32Subnormal = 1024, kBf16Convert = 2048, kRowXor = 4096,
-    kRowSum = 8192
+    kRowSum = 8192, kWeightTerms = 16384
 };
 
 // bf16 rounding cases: ties to even (both ways), a carry into the exponent,
@@ -27,6 +29,30 @@ __constant__ uint32_t kBf16Cases[16] = {
 // A[i][k] = (i + 2k) % 5 - 2, B[k][j] = (3k + j) % 7 - 3 (all exact)
 __device__ __forceinline__ float Aval(int i, int k) { return (float)((i + 2 * k) % 5 - 2); }
 __device__ __forceinline__ float Bval(int k, int j) { return (float)((3 * k + j) % 7 - 3); }
+
+// Whether the terms of weights with 24 significant bits add up to them: from
+// 2^lo to 2^hi, exactly, or to `off` below the exponents where they must be
+template <bool BF>
+__device__ bool weight_terms_hold(int l, int lo, int exact_from, int hi, float off) {
+    bool ok = true;
+    uint32_t r = 0x9e3779b9u * (uint32_t)(l + 1);
+    for (int e = lo; e <= hi; ++e) {
+        float x[2], left[2];
+        for (int i = 0; i < 2; ++i) {
+            r = r * 1664525u + 1013904223u;
+            x[i] = __builtin_ldexpf(1.0f + (float)((r >> 9) | 1u) * 0x1p-23f, e);  // odd last bit
+            left[i] = x[i];
+        }
+        uint32_t t[WeightTerms<BF>::n];
+        WeightTerms<BF>::split(left[0], left[1], t);
+        for (int i = 0; i < 2; ++i) {
+            float rest = x[i];
+            for (int u = 0; u < WeightTerms<BF>::n; ++u) rest -= half_to_f32<BF>((uint16_t)(t[u] >> (16 * i)));
+            ok &= fabsf(rest) <= (e >= exact_from ? 0.0f : off);
+        }
+    }
+    return ok;
+}
 
 __global__ void __launch_bounds__(64) selftest_kernel(int* fail) {
     __shared__ __attribute__((aligned(16))) float sc[16];
@@ -65,6 +91,9 @@ __global__ void __launch_bounds__(64) selftest_kernel(int* fail) {
         for (int i = 0; i < 16; ++i) ref += (float)(3 * (16 * grp + i) + 1);
         if (row_sum16((float)(3 * l + 1)) != ref) bad |= kRowSum;
     }
+    // fp16: whole down to a last bit of 2^-24, then off by half of that
+    if (!weight_terms_hold<false>(l, -30, -1, 14, 0x1p-25f) || !weight_terms_hold<true>(l, -80, -80, 14, 0.0f))
+        bad |= kWeightTerms;
     // 16x16x32 f16: A lane (row l%16, k = 8*(l/16) + e), D rows 4*(l/16)+i, col l%16
     {
         f16x8 a, b;
