@@ -148,7 +148,7 @@ SELFTEST_CHECKS = {1: "sum over rows", 2: "max over rows", 4: "LDS gather",
                    1024: "mfma 16x16x32 f16 subnormal operands",
                    2048: "bf16 conversion instruction vs the integer rounding rule",
                    4096: "16-lane DPP xor exchanges", 8192: "16-lane DPP row sum",
-                   16384: "16-bit terms of a weight"}
+                   16384: "16-bit terms of a weight", 32768: "table sums of squared centroids"}
 
 
 def selftest():

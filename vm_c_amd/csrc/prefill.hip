@@ -150,7 +150,7 @@ int tq_prefill_tiled(void* out, const void* query, const void* kv_cache, const i
     if (!cfg->key_fp8) {
         const TQTables& tab = tq_tables(kD, cfg->key_quant_bits);
         for (int i = 0; i < 16; ++i) prm.cent[i] = i < tab.n_centroids ? tab.centroids[i] : 0.0f;
-        prm.sq_unit = tq_fixed24_planes(prm.cent, cfg->key_quant_bits, prm.sq_plane);
+        prm.sq_unit = tq_square_planes(prm.cent, cfg->key_quant_bits, prm.sq_plane);
         prm.rot_c = tab.rot_c;
     }
     prm.fp8_e4b15 = cfg->fp8_e4b15 ? 1 : 0;

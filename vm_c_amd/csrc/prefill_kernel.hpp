@@ -72,7 +72,7 @@ struct PrefillParams {
     int q_bf16;          // paged: q / out (TurboQuant: and the stored halves) are bf16
     // TurboQuant slots: Lloyd-Max centroids, 1 / sqrt(d), field offsets
     float cent[16];
-    uint32_t sq_plane[12];  // cent[i]^2 / sq_unit, rounded: byte planes (tq_lut.hpp)
+    uint32_t sq_plane[16];  // cent[i]^2 / sq_unit, rounded: byte planes (tq_lut.hpp)
     float sq_unit;
     float rot_c;
     int mse_bytes, key_packed, val_data;
@@ -120,7 +120,7 @@ struct PrefillLds {
     float scratch[2][NW][32];            // [alpha, l][wave][row]
     alignas(8) uint8_t wide[NSLOT][NW];  // bf16: wave w's V rows of the tile need the exact mode
     float tq_base[2][16];                // TurboQuant: key centroids, value codes 0 .. 15
-    uint32_t tq_sq[12];                  // squared centroids, 24-bit fixed point, as byte planes
+    uint32_t tq_sq[16];                  // squared centroids, 32-bit fixed point, as byte planes
     alignas(16) uint8_t vtr[NSLOT][kD * BN * 2];  // [slot][dim][kv position] fp16 V^T
     uint8_t tile[NSLOT][2][BN * 256];             // [slot][K, V][row][position]
 };
@@ -271,7 +271,7 @@ prefill_kernel(PrefillParams p) {
             qb[s] = as_v8<V8>(u32x4{wd[0], wd[1], wd[2], wd[3]});
         }
         if (tid < 32) lds.tq_base[tid >> 4][tid & 15] = tid < 16 ? p.cent[tid] : (float)(tid & 15);
-        if (tid < 12) lds.tq_sq[tid] = p.sq_plane[tid];
+        if (tid < 16) lds.tq_sq[tid] = p.sq_plane[tid];
         __syncthreads();
     }
 
@@ -427,9 +427,10 @@ prefill_kernel(PrefillParams p) {
                 // C[i] * norm / ||C[codes]|| (C[i] * norm without the norm
                 // correction), or i * scale + zero.  They are computed once per
                 // lane and block, split into low and high bytes, and looked up
-                // four codes at a time by byte permutes (tq_lut.hpp): 1497 us
-                // on 2048 tokens over a 30720-token prefix of 3-bit slots, where
-                // one LDS gather, multiply and conversion per code took 1687 us.
+                // four codes at a time by byte permutes (tq_lut.hpp): 1403 us
+                // on 2048 tokens over a 30720-token prefix of 3-bit slots (4-bit
+                // 1547), of which 1497 against 1687 came with the tables alone:
+                // one LDS gather, multiply and conversion per code before.
                 constexpr int NB = TKB > TVB ? TKB : TVB;
                 using Lut = TqLut<NB>;
                 const bool kpart = lane < 32;
@@ -471,21 +472,16 @@ prefill_kernel(PrefillParams p) {
                             sel[j][u] = NB == 3 ? s3[u] : TKB == 4 ? s4[u] : kpart ? s3[u] : s4[u];
                     }
                 }
-                // ||C[codes]||^2 as a sum of 24-bit fixed-point squares (exact
+                // ||C[codes]||^2 as a sum of 32-bit fixed-point squares (exact
                 // integers; the four lanes of a quad hold the row's four blocks)
                 float f = half_f(hw2), add = 0.0f;
                 {
-                    uint32_t sq[TKB == 4 ? 12 : 6];
+                    constexpr int NS = 1 << TKB;  // dwords: 2^TKB entries
+                    uint32_t sq[NS];
 #pragma unroll
-                    for (int i = 0; i < (TKB == 4 ? 12 : 6); ++i) sq[i] = lds.tq_sq[i];
-                    uint32_t ss = 0;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-#pragma unroll
-                        for (int u = 0; u < 2; ++u) TqLut<TKB>::add_fixed24(sel[j][u], sq, ss);
-                    ss += (uint32_t)__shfl_xor((int)ss, 1, kWave);
-                    ss += (uint32_t)__shfl_xor((int)ss, 2, kWave);
-                    const float nrm = __builtin_amdgcn_rsqf(__builtin_fmaf((float)ss, p.sq_unit, 1e-16f));
+                    for (int i = 0; i < NS; ++i) sq[i] = lds.tq_sq[i];
+                    const float nrm = __builtin_amdgcn_rsqf(
+                        __builtin_fmaf(tq_row_squares<TKB>(sel, sq, lane), p.sq_unit, 1e-16f));
                     if (kpart) {
                         f *= p.norm_corr ? nrm : 1.0f;
                     } else {

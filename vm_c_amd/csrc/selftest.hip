@@ -2,11 +2,13 @@
 // on: cross-row reductions, the wave-private LDS gathers, the operand /
 // result layouts of the MFMA shapes used (16x16x32 f16/bf16, 16x16x16 f16,
 // 32x32x16 f16/bf16), exact fp16 subnormal operands in the 16x16x16 MFMA,
-// the bf16 conversion instruction, the 16-lane DPP exchanges and what the
-// 16-bit terms of a weight leave out.  One wave,
+// the bf16 conversion instruction, the 16-lane DPP exchanges, what the 16-bit
+// terms of a weight leave out and the table sums of squared centroids.  One wave,
 // fixed inputs (small integers where arithmetic is checked), every lane
 // compares its own results with the expected values.
+#include "tq_lut.hpp"
 #include "vmc_common.hpp"
+#include "vmc_tq.hpp"
 #include "weight_terms.hpp"
 
 namespace vmc {
@@ -16,7 +18,7 @@ enum {
     kSumGroups = 1, kMaxGroups = 2, kGather = 4, kMfma16x32 = 8, kMfma16x16 = 16,
     kMfma32x16 = 32, kMfma16x32bf = 64, kMfma32x16bf = 128, kMfma16x16Subnormal = 256,
     kGatherDiag = 512, kMfma16x32Subnormal = 1024, kBf16Convert = 2048, kRowXor = 4096,
-    kRowSum = 8192, kWeightTerms = 16384
+    kRowSum = 8192, kWeightTerms = 16384, kSquareSum = 32768
 };
 
 // bf16 rounding cases: ties to even (both ways), a carry into the exponent,
@@ -54,7 +56,33 @@ __device__ bool weight_terms_hold(int l, int lo, int exact_from, int hi, float o
     return ok;
 }
 
-__global__ void __launch_bounds__(64) selftest_kernel(int* fail) {
+// The tables of one code width, and whether rows of 128 codes (one code, then
+// codes that start at it and go on by 1, 2 and 3) sum to their squares within fp32's
+// own rounding: half an entry's last unit, the sum's, the unit's and the
+// product's, 4 x 2^-24 of the sum
+struct SquareTab {
+    float cent[16], unit;
+    uint32_t planes[16];
+};
+template <int BITS>
+__device__ bool square_sums_hold(const SquareTab& t, int l) {
+    constexpr uint32_t N = 1u << BITS;
+    bool ok = true;
+    for (uint32_t step = 0; step < 4; ++step) {
+        uint32_t sel[4][2];
+        double ref = 0.0;
+        for (uint32_t i = 0; i < 32; ++i) {
+            const uint32_t code = ((uint32_t)((l & 31) >> 2) + step * i) % N;
+            if ((i & 3) == 0) sel[i >> 3][(i >> 2) & 1] = 0;
+            sel[i >> 3][(i >> 2) & 1] |= (l < 32 ? code : N - 1 - code) << (8 * (i & 3));  // lanes 32 on: not counted
+            ref += 4.0 * (double)t.cent[code] * t.cent[code];
+        }
+        ok &= fabs((double)(tq_row_squares<BITS>(sel, t.planes, l) * t.unit) - ref) <= 0x1p-22 * ref;
+    }
+    return ok;
+}
+
+__global__ void __launch_bounds__(64) selftest_kernel(int* fail, SquareTab t3, SquareTab t4) {
     __shared__ __attribute__((aligned(16))) float sc[16];
     const int l = threadIdx.x, r16 = l & 15, grp = l >> 4;
     int bad = 0;
@@ -94,6 +122,7 @@ __global__ void __launch_bounds__(64) selftest_kernel(int* fail) {
     // fp16: whole down to a last bit of 2^-24, then off by half of that
     if (!weight_terms_hold<false>(l, -30, -1, 14, 0x1p-25f) || !weight_terms_hold<true>(l, -80, -80, 14, 0.0f))
         bad |= kWeightTerms;
+    if (!square_sums_hold<3>(t3, l) || !square_sums_hold<4>(t4, l)) bad |= kSquareSum;
     // 16x16x32 f16: A lane (row l%16, k = 8*(l/16) + e), D rows 4*(l/16)+i, col l%16
     {
         f16x8 a, b;
@@ -184,6 +213,14 @@ __global__ void __launch_bounds__(64) selftest_kernel(int* fail) {
     atomicOr(fail, bad);
 }
 
+SquareTab square_tab(int bits) {
+    SquareTab t = {};
+    const TQTables& tab = tq_tables(128, bits);
+    for (int i = 0; i < tab.n_centroids; ++i) t.cent[i] = tab.centroids[i];
+    t.unit = tq_square_planes(t.cent, bits, t.planes);
+    return t;
+}
+
 }  // namespace
 }  // namespace vmc
 
@@ -196,7 +233,7 @@ extern "C" int vmc_selftest(void) {
     int rc = VMC_OK;
     if (hipMemset(d, 0, sizeof(int)) != hipSuccess) rc = VMC_EIO;
     if (rc == VMC_OK) {
-        hipLaunchKernelGGL(vmc::selftest_kernel, dim3(1), dim3(64), 0, 0, d);
+        hipLaunchKernelGGL(vmc::selftest_kernel, dim3(1), dim3(64), 0, 0, d, vmc::square_tab(3), vmc::square_tab(4));
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
             hipMemcpy(&h, d, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
             rc = VMC_EIO;

@@ -87,35 +87,60 @@ struct TqLut {
         const uint32_t l = look(lo, s, s7, m8), h = look(hi, s, s7, m8);
         return u32x2{__builtin_amdgcn_perm(h, l, 0x05010400u), __builtin_amdgcn_perm(h, l, 0x07030602u)};
     }
-    // acc += the 24-bit entries of four codes; planes: 3 x kP dwords, low bytes first
-    static __device__ __forceinline__ void add_fixed24(uint32_t s, const uint32_t* planes, uint32_t& acc) {
+    // acc[b] += byte b of the 32-bit entries of four codes; planes: 4 x kP
+    // dwords, low bytes first
+    static __device__ __forceinline__ void add_squares(uint32_t s, const uint32_t* planes, uint32_t (&acc)[4]) {
         const uint32_t s7 = low3(s), m8 = bit3(s);
-        const uint32_t b0 = look(planes, s, s7, m8), b1 = look(planes + kP, s, s7, m8),
-                       b2 = look(planes + 2 * kP, s, s7, m8);
-        acc = __builtin_amdgcn_udot4(b0, 0x01010101u, acc, false);
-        acc += __builtin_amdgcn_udot4(b1, 0x01010101u, 0u, false) << 8;
-        acc += __builtin_amdgcn_udot4(b2, 0x01010101u, 0u, false) << 16;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            acc[b] = __builtin_amdgcn_udot4(look(planes + b * kP, s, s7, m8), 0x01010101u, acc[b], false);
     }
 };
 
+// The sum of a K row's 128 entries in units, for lanes 0 .. 31 and 32 on alike:
+// sel holds 32 codes of it in each of four lanes below 32 (a quad), one a byte.
+// The lane 32 on takes half of them (its own are V's): 2048 tokens over a
+// 30720-token prefix of 4-bit slots 1547 us, 1689 with every lane looking up all
+// 32.  Integers keep the sum exact (each half word's below 2^23) up to the one
+// rounding here.
+template <int BITS>
+__device__ __forceinline__ float tq_row_squares(const uint32_t (&sel)[4][2], const uint32_t* planes, int lane) {
+    uint32_t acc[4] = {};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t mine = sel[j][0], theirs = sel[j][1];
+        swap_pair32(mine, theirs);  // lanes 32 on: sel[j][1] of 32 lanes below
+        TqLut<BITS>::add_squares(mine, planes, acc);
+    }
+    uint32_t w[2] = {(acc[1] << 8) + acc[0], (acc[3] << 8) + acc[2]};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        w[i] += row_xor_u32<1>(w[i], lane);
+        w[i] += row_xor_u32<2>(w[i], lane);
+        uint32_t o = w[i];
+        swap_pair32(w[i], o);
+        w[i] += o;
+    }
+    return __builtin_fmaf((float)w[1], 65536.0f, (float)w[0]);
+}
+
 }  // namespace
 
-// c[i]^2 of the 2^bits centroids in 24-bit fixed point, as byte planes
-// (3 x 2^bits / 4 dwords).  Returns the unit: the largest square is 2^24 - 1
-// units, so a sum of 128 stays below 2^31.  Each entry is off by half a unit
-// at most and the sum by 6 units or so (64 at most), 2^-22 (2^-18) of the
-// largest square, where the sum is about 27 (3-bit) or 17 (4-bit) of them:
-// the rounding of a 128-term fp32 sum.
-inline float tq_fixed24_planes(const float* cent, int bits, uint32_t* planes) {
+// c[i]^2 of the 2^bits centroids in 32-bit fixed point, as byte planes
+// (2^bits entries: 2^bits dwords).  Returns the unit: the largest square is
+// 2^32 - 1 of them.  An entry is off by half a unit at most, 2^-24 of the
+// smallest square (4-bit; 3-bit 2^-28): no more than a squared fp32 centroid's
+// own rounding, and the sum itself is exact where fp32 rounds at each term.
+inline float tq_square_planes(const float* cent, int bits, uint32_t* planes) {
     const int n = 1 << bits, np = n / 4;
     double mx = 0.0;
     for (int i = 0; i < n; ++i) mx = fmax(mx, (double)cent[i] * cent[i]);
-    const float unit = (float)(mx / 16777215.0 * (1.0 + 1e-7));
-    for (int i = 0; i < 3 * np; ++i) planes[i] = 0;
+    const float unit = (float)(mx / 4294967295.0 * (1.0 + 1e-7));
+    for (int i = 0; i < 4 * np; ++i) planes[i] = 0;
     for (int i = 0; i < n; ++i) {
-        uint32_t q = (uint32_t)(int64_t)rint((double)cent[i] * cent[i] / (double)unit);
-        if (q > 0xffffffu) q = 0xffffffu;
-        for (int b = 0; b < 3; ++b) planes[b * np + i / 4] |= ((q >> (8 * b)) & 255u) << (8 * (i & 3));
+        double q = rint((double)cent[i] * cent[i] / (double)unit);
+        if (q > 4294967295.0) q = 4294967295.0;
+        for (int b = 0; b < 4; ++b) planes[b * np + i / 4] |= (((uint32_t)q >> (8 * b)) & 255u) << (8 * (i & 3));
     }
     return unit;
 }
