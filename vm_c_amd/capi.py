@@ -7,8 +7,6 @@ if the library is missing or a call fails, this raises.
 import ctypes as C
 import os
 
-import torch
-
 PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG, "libvmc_attn.so")
 
@@ -122,23 +120,41 @@ def _check(rc, what):
 # A decode step is two calls of a few microseconds of GPU time each, so what a
 # call costs here counts: addresses go to ctypes as plain integers (the
 # argtypes make them pointers), and the current stream's handle is asked for
-# without a torch.cuda.Stream object around it.
+# without a torch.cuda.Stream object around it where this torch can.  torch is
+# imported by the first call that takes tensors: the host-only ones do without.
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def _bind_current_stream():
+    global _current_stream
+    import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        _current_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    else:
+        _current_stream = lambda: raw(torch.cuda.current_device())  # noqa: E731
+    return _current_stream()
+
+
+_current_stream = _bind_current_stream
+
+
 def _stream(stream=None):
-    if stream is not None:
-        return stream.cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return _current_stream() if stream is None else stream.cuda_stream
+
+
+_dtype_codes = {}
 
 
 def _dtype_code(t):
-    if t.dtype == torch.float16:
-        return DTYPE_F16
-    if t.dtype == torch.bfloat16:
-        return DTYPE_BF16
-    raise VmcError(f"unsupported dtype {t.dtype}")
+    if not _dtype_codes:
+        import torch
+        _dtype_codes.update({torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16})
+    code = _dtype_codes.get(t.dtype)
+    if code is None:
+        raise VmcError(f"unsupported dtype {t.dtype}")
+    return code
 
 
 SELFTEST_CHECKS = {1: "sum over rows", 2: "max over rows", 4: "LDS gather",
@@ -229,11 +245,11 @@ def paged_decode_workspace_size(batch, num_heads, num_kv_heads, head_dim=128, ma
 def paged_attention_decode(out, query, key_cache, value_cache, block_tables, seq_lens,
                            num_kv_heads, scale, block_size=16, kv_format=KV_F16,
                            layout=LAYOUT_NHD, workspace=None, max_splits=0, stream=None):
-    import torch
     B, Hq, D = query.shape
     max_blocks = block_tables.shape[1]
     ws_bytes = paged_decode_workspace_size(B, Hq, num_kv_heads, D, max_blocks, block_size, max_splits)
     if workspace is None:
+        import torch
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=query.device)
     rc = load().vmc_paged_attention_decode(
         _ptr(out), _ptr(query), _ptr(key_cache), _ptr(value_cache), _ptr(block_tables),
@@ -260,12 +276,12 @@ def turboquant_decode_workspace_size(batch, num_heads, num_kv_heads, head_dim=12
 
 def turboquant_decode_attention(out, query, kv_cache, block_tables, seq_lens, num_kv_heads, scale,
                                 cfg, block_size=16, workspace=None, max_splits=0, stream=None):
-    import torch
     B, Hq, D = query.shape
     max_blocks = block_tables.shape[1]
     ws_bytes = turboquant_decode_workspace_size(B, Hq, num_kv_heads, D, max_blocks, block_size,
                                                 max_splits)
     if workspace is None:
+        import torch
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=query.device)
     rc = load().vmc_turboquant_decode_attention(
         _ptr(out), _ptr(query), _ptr(kv_cache), _ptr(block_tables), _ptr(seq_lens), B, Hq,
@@ -343,11 +359,11 @@ def paged_attention_prefill(out, query, key_cache, value_cache, block_tables, to
                             layout=LAYOUT_NHD, workspace=None, max_splits=1, stream=None):
     """query/out [T][Hq][D]: token t attends positions 0 .. token_positions[t] of
     sequence token_to_seq[t] in the paged cache."""
-    import torch
     T, Hq, D = query.shape
     max_blocks = block_tables.shape[1]
     ws_bytes = paged_decode_workspace_size(T, Hq, num_kv_heads, D, max_blocks, block_size, max_splits)
     if workspace is None and ws_bytes > 0:
+        import torch
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
     rc = load().vmc_paged_attention_prefill(
         _ptr(out), _ptr(query), _ptr(key_cache), _ptr(value_cache), T, Hq, num_kv_heads, D, scale,
