@@ -1,8 +1,10 @@
-"""The ctypes binding's host side: what it needs of torch."""
+"""The ctypes binding's host side: what it needs of torch, and the workspaces
+that it allocates for a call on another stream."""
 import subprocess
 import sys
 import types
 
+import numpy as np
 import pytest
 
 from conftest import ROOT
@@ -31,3 +33,37 @@ def test_current_stream(monkeypatch, raw):
         monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
     assert [capi._stream(), capi._stream()] == [103 if raw else 7] * 2
     assert capi._stream(types.SimpleNamespace(cuda_stream=11)) == 11
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_own_workspace_on_another_stream(dev, d):
+    """A decode on a busy side stream without a workspace: memory that the
+    current stream gets after the call is not the one the call still writes its
+    partial rows to."""
+    import torch
+    from vm_c_amd import capi
+    B, H, L = 2, 8, 4096
+    q = torch.randn(B, H, d, device=dev).half()
+    kc, vc = (torch.randn(B * L * H * d, device=dev).half().view(torch.uint8) for _ in range(2))
+    bt = torch.from_numpy(np.arange(B * L // 16, dtype=np.int32).reshape(B, -1)).to(dev)
+    lens = torch.full((B,), L, dtype=torch.int32, device=dev)
+    out, ref = torch.empty_like(q), torch.empty_like(q)
+
+    def run(o, stream=None):
+        capi.paged_attention_decode(o, q, kc, vc, bt, lens, H, d ** -0.5, stream=stream)
+
+    run(ref)
+    size = capi.paged_decode_workspace_size(B, H, H, d, L // 16)
+    a = torch.randn(8192, 8192, device=dev).half()
+    c = a @ a
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    with torch.cuda.stream(side):
+        for _ in range(20):  # about 1 ms each
+            torch.matmul(a, a, out=c)
+    run(out, side)
+    mine = torch.full((size,), 0xff, dtype=torch.uint8, device=dev)
+    torch.cuda.synchronize()
+    assert (mine == 0xff).all() and torch.equal(out, ref)

@@ -157,6 +157,17 @@ def _dtype_code(t):
     return code
 
 
+def _workspace(nbytes, like, stream):
+    """Device memory for one call on `stream`.  The caller drops it on return, while
+    the call may still be running: the allocator must not hand it to the
+    current stream's work before `stream` is past the call."""
+    import torch
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=like.device)
+    if stream is not None:
+        ws.record_stream(stream)
+    return ws
+
+
 SELFTEST_CHECKS = {1: "sum over rows", 2: "max over rows", 4: "LDS gather",
                    8: "mfma 16x16x32 f16", 16: "mfma 16x16x16 f16", 32: "mfma 32x32x16 f16",
                    64: "mfma 16x16x32 bf16", 128: "mfma 32x32x16 bf16",
@@ -249,8 +260,7 @@ def paged_attention_decode(out, query, key_cache, value_cache, block_tables, seq
     max_blocks = block_tables.shape[1]
     ws_bytes = paged_decode_workspace_size(B, Hq, num_kv_heads, D, max_blocks, block_size, max_splits)
     if workspace is None:
-        import torch
-        workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=query.device)
+        workspace = _workspace(max(ws_bytes, 1), query, stream)
     rc = load().vmc_paged_attention_decode(
         _ptr(out), _ptr(query), _ptr(key_cache), _ptr(value_cache), _ptr(block_tables),
         _ptr(seq_lens), B, Hq, num_kv_heads, D, block_size, max_blocks, scale,
@@ -281,8 +291,7 @@ def turboquant_decode_attention(out, query, kv_cache, block_tables, seq_lens, nu
     ws_bytes = turboquant_decode_workspace_size(B, Hq, num_kv_heads, D, max_blocks, block_size,
                                                 max_splits)
     if workspace is None:
-        import torch
-        workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=query.device)
+        workspace = _workspace(max(ws_bytes, 1), query, stream)
     rc = load().vmc_turboquant_decode_attention(
         _ptr(out), _ptr(query), _ptr(kv_cache), _ptr(block_tables), _ptr(seq_lens), B, Hq,
         num_kv_heads, D, scale, block_size, max_blocks, C.byref(cfg), _dtype_code(query),
@@ -363,8 +372,7 @@ def paged_attention_prefill(out, query, key_cache, value_cache, block_tables, to
     max_blocks = block_tables.shape[1]
     ws_bytes = paged_decode_workspace_size(T, Hq, num_kv_heads, D, max_blocks, block_size, max_splits)
     if workspace is None and ws_bytes > 0:
-        import torch
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
+        workspace = _workspace(ws_bytes, query, stream)
     rc = load().vmc_paged_attention_prefill(
         _ptr(out), _ptr(query), _ptr(key_cache), _ptr(value_cache), T, Hq, num_kv_heads, D, scale,
         block_size, max_blocks, _ptr(block_tables), _ptr(token_to_seq), _ptr(token_positions),
