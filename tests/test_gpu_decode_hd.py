@@ -112,6 +112,39 @@ def test_prefill_rows(dev, d, splits):
     _close(got, ref, ulp)
 
 
+# rows enough that a merge workgroup takes several heads and scans more than 256
+# lengths, and the last and first counts on either side of one range per row
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("rows", [300, 1023, 1024])
+def test_many_rows(dev, d, rows):
+    import torch
+    from vm_c_amd import capi
+    w, _, pages, _, Hkv, scale, kw = _setup(dev, d, (14, 2), BF16, "bf16", False, lens=[300, 150, 7], seed=14)
+    rng = np.random.default_rng(rows)
+    seq = np.sort(rng.integers(0, 3, rows)).astype(np.int32)
+    pos = (rng.random(rows) * np.asarray([300, 150, 7])[seq]).astype(np.int32)
+    pos[::50] = -1  # rows without keys
+    g = torch.Generator().manual_seed(d)
+    Q = torch.randn((rows, 14, d), generator=g).to(dev).to(torch.bfloat16)
+    ts, tp = torch.from_numpy(seq).to(dev), torch.from_numpy(pos).to(dev)
+    got, ref, ulp = _both(Q, lambda o: capi.paged_attention_prefill(o, Q, *pages, ts, tp, Hkv, scale, max_splits=0,
+                                                                    **kw))
+    _close(got, ref, ulp)
+    assert (got[::50] == 0).all()
+
+
+# tables of as many pages as one wave takes without a split, and one more
+@pytest.mark.parametrize("d,wide", [(64, 8), (64, 9), (256, 4), (256, 5)])
+def test_narrow_table(dev, d, wide):
+    from vm_c_amd import capi
+    w, Q, pages, lens, Hkv, scale, kw = _setup(dev, d, (8, 2), F16, "f16", False, lens=[16 * wide, 1, 0, 16 * wide - 17],
+                                               seed=15)
+    assert pages[2].shape[1] == wide
+    got, ref, ulp = _both(Q, lambda o: capi.paged_attention_decode(o, Q, *pages, lens, Hkv, scale, **kw))
+    _close(got, ref, ulp)
+    assert (got[2] == 0).all()
+
+
 # infinities and NaNs: V of a key whose weight is 0 (alone, and among 20 pages
 # of such keys, so that whole pieces are), V of one that counts (the last one
 # too), K, q; scores far enough apart that weights underflow.  Whole sequences, and ones

@@ -442,43 +442,58 @@ __global__ void __launch_bounds__(1024) decode_merge_kernel(DecodeParams p) {
 // weights 2^(s - m), s the score in log2 units, whichever loop wrote the row;
 // no key: m = -inf, l = 0).  A piece of weight 0 adds nothing, also where its o
 // holds an infinity: the key that brought it has weight 0 in the whole row (an
-// l that is NaN, from a score that is, stays one).  Four waves per (sequence,
-// query head): grid (B, Hq), 256 threads; wave w takes pieces w, w + 4, ...
-// (sixteen rows in flight, so 64 pieces cost one round of loads), lane l dims
-// l D / 64 .. ; the four partial sums meet in LDS.
+// l that is NaN, from a score that is, stays one).
+// Grid (B, merge_rows_y), 256 threads: a workgroup finds its sequence's pages in
+// one scan over the lengths, then takes query heads blockIdx.y, + gridDim.y, ..
+// of it.  Wave w takes pieces w, w + 4, ... (sixteen rows in flight, so 64 pieces
+// cost one round of loads), lane l dims l D / 64 .. ; the four partial sums meet
+// in LDS.  The scan is what many rows cost: with a workgroup per (row, head) and
+// one load of 64 lengths after another, 1000 rows of up to 300 keys (14 / 2
+// heads of 64, bf16) took 99 us with their split pass, now 71 (8 / 1 heads of 256:
+// 105, 83).
 template <int D>
 __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) {
     constexpr int NV = D / 64;
+    static_assert(NV == 1 || NV == 4, "head_dim 64 or 256");
     typedef float fv __attribute__((ext_vector_type(NV)));
     __shared__ __attribute__((aligned(16))) float red[4][D + 4];
-    const int b = blockIdx.x, hq = blockIdx.y;
+    const int b = blockIdx.x;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int carry = 0, ps_b = 0, pg_b = 0;
-    for (int b0 = 0; b0 < p.B; b0 += 64) {
-        int L = 0;
-        const int pg = b0 + lane < p.B ? seq_pages(p, b0 + lane, &L) : 0;
-        const int incl = wave_incl_scan(pg, lane);
-        if (b >= b0 && b < b0 + 64) {  // uniform over the wave
-            pg_b = __builtin_amdgcn_readlane(pg, b - b0);
-            ps_b = carry + __builtin_amdgcn_readlane(incl, b - b0) - pg_b;
+    for (int b0 = 0; b0 < p.B; b0 += 256) {
+        int pgs[4] = {};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {  // four loads in flight
+            int L = 0;
+            if (u > 0 && b0 + 64 * u >= p.B) break;  // uniform
+            const int r = b0 + 64 * u + lane, n = seq_pages(p, min(r, p.B - 1), &L);
+            pgs[u] = r < p.B ? n : 0;
         }
-        carry += __builtin_amdgcn_readlane(incl, 63);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int bu = b0 + 64 * u;
+            if (bu >= p.B) break;  // uniform
+            const int incl = wave_incl_scan(pgs[u], lane);
+            if (b >= bu && b < bu + 64) {  // uniform
+                pg_b = __builtin_amdgcn_readlane(pgs[u], b - bu);
+                ps_b = carry + __builtin_amdgcn_readlane(incl, b - bu) - pg_b;
+            }
+            carry += __builtin_amdgcn_readlane(incl, 63);
+        }
     }
     const int T = carry;
-    uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + ((int64_t)b * p.Hq + hq) * D + NV * lane;
-    auto put = [&](const fv& x) __attribute__((always_inline)) {
+    auto put = [&](int hq, const fv& x) __attribute__((always_inline)) {
+        uint16_t* orow = reinterpret_cast<uint16_t*>(p.out) + ((int64_t)b * p.Hq + hq) * D + NV * lane;
         uint16_t h[NV];
 #pragma unroll
         for (int e = 0; e < NV; ++e) h[e] = p.q_bf16 ? f32_to_bf16_bits(x[e]) : f32_to_f16_bits(x[e]);
         if constexpr (NV == 4)
             *reinterpret_cast<u32x2*>(orow) = u32x2{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16)};
-        else if constexpr (NV == 2)
-            *reinterpret_cast<uint32_t*>(orow) = h[0] | ((uint32_t)h[1] << 16);
         else
             orow[0] = h[0];
     };
     if (pg_b == 0) {
-        if (wave == 0) put(fv(0.0f));
+        for (int hq = blockIdx.y + gridDim.y * wave; hq < p.Hq; hq += 4 * gridDim.y) put(hq, fv(0.0f));
         return;
     }
     const int n = effective_wgs(p, T, p.grid);
@@ -486,68 +501,71 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
     if (w0 == w1) return;  // written by its range
     const int nseg = w1 - w0 + 1;
     const int64_t rs = (int64_t)p.Hq * (D + 4);
-    auto row = [&](int s) {  // piece s = range w0 + s
-        const int64_t slot = s == 0 ? 2 * w0 + 1 : 2 * (w0 + s);
-        return p.part + slot * rs + (int64_t)hq * (D + 4);
-    };
-    float M = kNegInf, L = 0.0f;
-    fv acc = fv(0.0f);
-    for (int s0 = wave; s0 < nseg; s0 += 64) {
-        fv o[16];
-        float2 ml[16];
+    for (int hq = blockIdx.y; hq < p.Hq; hq += gridDim.y) {
+        if (hq != (int)blockIdx.y) __syncthreads();  // the last head's sums are read
+        auto row = [&](int s) {  // piece s = range w0 + s
+            const int64_t slot = s == 0 ? 2 * w0 + 1 : 2 * (w0 + s);
+            return p.part + slot * rs + (int64_t)hq * (D + 4);
+        };
+        float M = kNegInf, L = 0.0f;
+        fv acc = fv(0.0f);
+        for (int s0 = wave; s0 < nseg; s0 += 64) {
+            fv o[16];
+            float2 ml[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const float* r = row(min(s0 + 4 * u, nseg - 1));
-            ml[u] = *reinterpret_cast<const float2*>(r + D);
-            o[u] = *reinterpret_cast<const fv*>(r + NV * lane);
+            for (int u = 0; u < 16; ++u) {
+                const float* r = row(min(s0 + 4 * u, nseg - 1));
+                ml[u] = *reinterpret_cast<const float2*>(r + D);
+                o[u] = *reinterpret_cast<const fv*>(r + NV * lane);
+            }
+            float mx = M;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) mx = s0 + 4 * u < nseg ? fmaxf(mx, ml[u].x) : mx;
+            if (mx > M && M != kNegInf) {  // wave-uniform
+                const float f = __builtin_amdgcn_exp2f(M - mx);
+                const bool none = f == 0.0f && L == L;
+                L *= f;
+#pragma unroll
+                for (int e = 0; e < NV; ++e) acc[e] = none ? 0.0f : acc[e] * f;
+            }
+            M = mx;
+            const float Mu = M == kNegInf ? 0.0f : M;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const float wu = s0 + 4 * u < nseg ? __builtin_amdgcn_exp2f(ml[u].x - Mu) : 0.0f;
+                const bool none = wu == 0.0f && ml[u].y == ml[u].y;
+                L = __builtin_fmaf(ml[u].y, wu, L);
+#pragma unroll
+                for (int e = 0; e < NV; ++e) acc[e] = __builtin_fmaf(none ? 0.0f : o[u][e], wu, acc[e]);
+            }
         }
-        float mx = M;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) mx = s0 + 4 * u < nseg ? fmaxf(mx, ml[u].x) : mx;
-        if (mx > M && M != kNegInf) {  // wave-uniform
-            const float f = __builtin_amdgcn_exp2f(M - mx);
-            const bool none = f == 0.0f && L == L;
-            L *= f;
-#pragma unroll
-            for (int e = 0; e < NV; ++e) acc[e] = none ? 0.0f : acc[e] * f;
+        *reinterpret_cast<fv*>(&red[wave][NV * lane]) = acc;
+        if (lane == 0) {
+            red[wave][D] = M;
+            red[wave][D + 1] = L;
         }
-        M = mx;
-        const float Mu = M == kNegInf ? 0.0f : M;
+        __syncthreads();
+        if (wave != 0) continue;
+        float Mg = kNegInf;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const float wu = s0 + 4 * u < nseg ? __builtin_amdgcn_exp2f(ml[u].x - Mu) : 0.0f;
-            const bool none = wu == 0.0f && ml[u].y == ml[u].y;
-            L = __builtin_fmaf(ml[u].y, wu, L);
+        for (int w = 0; w < 4; ++w) Mg = fmaxf(Mg, red[w][D]);
+        const float Mgu = Mg == kNegInf ? 0.0f : Mg;
+        float Lg = 0.0f;
+        fv og = fv(0.0f);
 #pragma unroll
-            for (int e = 0; e < NV; ++e) acc[e] = __builtin_fmaf(none ? 0.0f : o[u][e], wu, acc[e]);
+        for (int w = 0; w < 4; ++w) {
+            const float f = red[w][D] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(red[w][D] - Mgu);
+            const bool none = f == 0.0f && red[w][D + 1] == red[w][D + 1];
+            Lg = __builtin_fmaf(red[w][D + 1], f, Lg);
+            const fv v = *reinterpret_cast<const fv*>(&red[w][NV * lane]);
+#pragma unroll
+            for (int e = 0; e < NV; ++e) og[e] = __builtin_fmaf(none ? 0.0f : v[e], f, og[e]);
         }
+        const float inv = Lg > 0.0f ? 1.0f / Lg : 0.0f;
+#pragma unroll
+        for (int e = 0; e < NV; ++e) og[e] *= inv;
+        put(hq, og);
     }
-    *reinterpret_cast<fv*>(&red[wave][NV * lane]) = acc;
-    if (lane == 0) {
-        red[wave][D] = M;
-        red[wave][D + 1] = L;
-    }
-    __syncthreads();
-    if (wave != 0) return;
-    float Mg = kNegInf;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) Mg = fmaxf(Mg, red[w][D]);
-    const float Mgu = Mg == kNegInf ? 0.0f : Mg;
-    float Lg = 0.0f;
-    fv og = fv(0.0f);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const float f = red[w][D] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(red[w][D] - Mgu);
-        const bool none = f == 0.0f && red[w][D + 1] == red[w][D + 1];
-        Lg = __builtin_fmaf(red[w][D + 1], f, Lg);
-        const fv v = *reinterpret_cast<const fv*>(&red[w][NV * lane]);
-#pragma unroll
-        for (int e = 0; e < NV; ++e) og[e] = __builtin_fmaf(none ? 0.0f : v[e], f, og[e]);
-    }
-    const float inv = Lg > 0.0f ? 1.0f / Lg : 0.0f;
-#pragma unroll
-    for (int e = 0; e < NV; ++e) og[e] *= inv;
-    put(og);
 }
 
 }  // namespace
@@ -555,6 +573,11 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
 // ------------------------------------------------------------------ host
 
 constexpr int kPpsMin = 2;
+
+// decode_merge_rows_kernel's workgroups per sequence: one for each query head
+// where there are few sequences, down to one for all of them from 2048 on (the
+// chip holds about as many workgroups)
+inline unsigned merge_rows_y(int B, int Hq) { return (unsigned)std::clamp(2048 / std::max(B, 1), 1, Hq); }
 
 // Launched workgroups for the flat layout: one resident wave of them (a
 // workgroup of Hkv waves at 2 waves per SIMD), fewer for small batches.

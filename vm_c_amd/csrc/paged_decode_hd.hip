@@ -10,7 +10,10 @@
 // 47 us, 3.7 TB/s); here
 //  * a wave is one (page range, KV head) unit: all G query heads share each
 //    page it reads, and the ranges (decode_plan.hpp) cut long sequences, so
-//    that every CU holds 12 (head_dim 64) or 8 units whatever the batch;
+//    that a CU holds 12 (head_dim 64) or 8 units whatever the batch, as far as
+//    the workspace has room for their partial rows (paged_decode_hd; the size
+//    query is by rows of 128 dims: at head_dim 256, 16/2 heads, 519 of the 1024
+//    ranges; 8/4 heads 259 of 512);
 //  * waves share nothing and meet no barrier: each finds its sequences by a
 //    scan of seq_lens, keeps 64 block-table entries in its lanes, and holds
 //    the next step's pages (32 tokens at head_dim 64, 16 at 256: 8 or 16 KB)
@@ -470,7 +473,8 @@ int launch_hd(DecodeParams& prm, hipStream_t stream) {
                        stream, prm);
     VMC_LAUNCH_CHECK();
     if (!prm.per_seq) {
-        hipLaunchKernelGGL(decode_merge_rows_kernel<D>, dim3(prm.B, prm.Hq), dim3(256), 0, stream, prm);
+        hipLaunchKernelGGL(decode_merge_rows_kernel<D>, dim3(prm.B, merge_rows_y(prm.B, prm.Hq)), dim3(256), 0,
+                           stream, prm);
         VMC_LAUNCH_CHECK();
     }
     return VMC_OK;
@@ -523,17 +527,25 @@ int paged_decode_hd(const GenArgs& a, int max_splits, void* ws, size_t ws_bytes,
     // Page ranges: 12 units per CU at head_dim 64, 8 at 256: one resident wave
     // of them (registers; 32 x 256 .. 8192 tokens at head_dim 64: 47.2 us,
     // 16 per CU 49.8, 24 per CU 53.0, 16 resident at 128 registers 57.6), no
-    // more than the workspace has partial rows for.  The
-    // entry points take a call without a workspace here, and one sized for
-    // rows of 128 dims: with room for fewer ranges than rows, each row is one
-    // range (no partial rows).
+    // more than the workspace has partial rows for.
+    // One range per row instead (no partial rows, no merge):
+    //  * where a wave walks the longest row the table allows in four steps, about
+    //    what the merge takes (100 rows of up to 50 keys, 32/8 heads of 64: 15.8
+    //    us in ranges, 5.4; 16/2 heads of 256: 19.8, 11.4);
+    //  * from 1024 rows on: a wave each fills the chip or half of it, while every
+    //    unit and merge workgroup would scan all rows' lengths (10,000 rows of up
+    //    to 300 keys, 32/8 heads of 64: 264 us; in ranges, with a merge workgroup
+    //    per row and head, 8.1 ms, and the one-wave kernel 4.1 ms);
+    //  * without room for as many ranges as rows or units.  The entry points take
+    //    a call without a workspace here, and one sized for rows of 128 dims.
     const int64_t pages = (int64_t)a.rows * a.max_blocks;
     int64_t n = std::max<int64_t>(1, (int64_t)num_cus() * (a.D == 64 ? 12 : 8) / a.Hkv);
     n = std::min<int64_t>(n, (pages + kPpsMin - 1) / kPpsMin);
     if (max_splits > 1) n = std::min<int64_t>(n, (int64_t)a.rows * max_splits);
     const int64_t room =
         ws && ((uintptr_t)ws & 15) == 0 ? (int64_t)(ws_bytes / ((size_t)2 * a.Hq * (a.D + 4) * sizeof(float))) : 0;
-    prm.per_seq = max_splits == 1 || pages > 0x7fffffff || room < std::min<int64_t>(n, a.rows) || room < 2;
+    prm.per_seq = max_splits == 1 || a.max_blocks <= (a.D == 64 ? 8 : 4) || a.rows >= 1024 || pages > 0x7fffffff ||
+                  room < std::min<int64_t>(n, a.rows) || room < 2;
     prm.grid = prm.per_seq ? a.rows : (int)std::min(n, room);
     const int fmt = a.src == GEN_F16 ? VMC_KV_F16 : a.src == GEN_BF16 ? VMC_KV_BF16 : a.src == GEN_Q8 ? VMC_KV_Q8_0 : VMC_KV_Q4_0;
     return a.D == 64 ? dispatch_hd<64>(prm, fmt, stream) : dispatch_hd<256>(prm, fmt, stream);
