@@ -376,7 +376,8 @@ int vmc_batch_token_rows(int32_t* row_seq, int32_t* row_pos, const int32_t* toke
  * vmc_reshape_and_cache, slot_mapping int64 [num_tokens]).
  * Limits: head_dim 64, 128 or 256 (64 and 256: the append by
  * vmc_reshape_and_cache, then the tiled kernel of those sizes, or a
- * one-wave-per-row kernel where q, out, K or V is not 16-byte aligned),
+ * one-wave-per-row kernel for steps of a few tokens and where q, out, K or V
+ * is not 16-byte aligned),
  * num_heads % num_kv_heads == 0.
  */
 int vmc_flash_attention_prefill(void* output, const void* query, const void* key,

@@ -29,7 +29,7 @@ def _inputs(dev, d, heads, seq_lens, bf16, seed=0):
 @pytest.mark.parametrize("d", [64, 256])
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("heads", [(2, 2), (4, 2), (8, 2), (7, 1), (16, 2)])
-@pytest.mark.parametrize("seq_lens", [[1], [64], [65, 63, 1, 1, 200], [31, 300, 33]])
+@pytest.mark.parametrize("seq_lens", [[1], [17], [25], [64], [65, 63, 1, 1, 200], [31, 300, 33]])
 def test_prefill(dev, d, bf16, heads, seq_lens):
     from vm_c_amd import capi
     q, k, v, pos, (qb, kb, vb, cu) = _inputs(dev, d, heads, seq_lens, bf16, seed=d + sum(seq_lens))
@@ -41,6 +41,23 @@ def test_prefill(dev, d, bf16, heads, seq_lens):
     ex = O.prefill_exact_rows(qb, kb, vb, cu, heads[1], sc, toks, hds, is_bf16=bf16).reshape(T, heads[0], d)
     err = np.abs(got.cpu().numpy() - ex)
     assert (err <= 2e-5 + ulp / 2 * np.abs(ex)).all(), float(err.max())
+
+
+# steps of enough workgroups for the eight-wave kernel (4, 2 and 1 heads a
+# workgroup), with an infinity in V of one KV head's early sequence
+@pytest.mark.parametrize("d", [64, 256])
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("heads", [(16, 2), (36, 6), (28, 4)])
+def test_prefill_long_steps(dev, d, bf16, heads):
+    from vm_c_amd import capi
+    hw = {8: 4, 6: 2, 7: 1}[heads[0] // heads[1]]
+    per_cu = 4 if d == 64 else 1
+    rows = (256 * per_cu + 1) * 32 * 4 // heads[0] + 64  # rows x heads / 128 workgroups of four waves
+    lens = [31, 300, 33, 65, 1, 200] * (rows // 630 + 1)
+    q, k, v, pos, _ = _inputs(dev, d, heads, lens, bf16, seed=hw)
+    v[40, 0, 3] = float("inf")
+    got, ref, ulp = _both(q, lambda o: capi.flash_attention_prefill(o, q, k, v, pos, heads[1], 1 / np.sqrt(d)))
+    _close(got, ref, ulp)
 
 
 # positions that are not 0 .. n-1 of contiguous sequences: every row's window

@@ -1,7 +1,7 @@
 // prefill_hd.hip -- causal flash-attention prefill of head_dim 64 and 256 over
 // this step's K/V rows, on MFMA.  The rows and their windows are
 // gen_attn_kernel's (generic_attn.hip: token t attends tokens t - pos[t] .. t),
-// which keeps operands that are not 16-byte aligned.
+// which keeps operands that are not 16-byte aligned and the shortest steps.
 //
 // What bounds it: the matrix cores (4 D flops per query, key and head; P V
 // counts three times, see below).  The one-wave-per-row kernel had no
@@ -10,7 +10,8 @@
 // TFLOP/s of the attention's own flops, 1.07 PFLOP/s on the matrix cores).
 // Workgroup = 8 waves = up to 4 query heads of one KV head x 32-row query
 // blocks, as prefill_kernel (prefill.hip), so a K/V tile of 64 keys in LDS
-// serves 256 query rows.  Tiles arrive by load-to-LDS transfers: three slots
+// serves 256 query rows; 4 waves and 128 rows where workgroups are few
+// (prefill_hd).  Tiles arrive by load-to-LDS transfers: three slots
 // at head_dim 64 (two tiles in flight), two at 256 (128 KB, one in flight).
 //   S^T[32 keys x 32 rows] = K . Q^T, O^T[D x 32 rows] += V^T . P^T on
 //   v_mfma_f32_32x32x16: a query row is one lane column in both, so its
@@ -35,6 +36,7 @@
 // exactly.  A row whose sums are not finite reruns key by key (gen_row): its
 // products met an infinity or a NaN, or bf16 V so large that weights of up to
 // 2^8 (the reference max lags by that much) overflow where weights of 1 do not.
+#include "device_cus.hpp"
 #include "generic_row.hpp"
 #include "prefill_dev.hpp"
 #include "prefill_hd.hpp"
@@ -43,8 +45,12 @@
 namespace vmc {
 namespace {
 
-constexpr int kHdW = 8;    // waves per workgroup
 constexpr int kHdBN = 64;  // keys per tile
+// Steps of no more rows stay with the one-wave-per-row kernel, whatever their
+// prompts (bf16, us there / here: head_dim 64, 14/2 heads, 8 rows 4.7 / 5.6, 17
+// rows 6.2 / 5.5; 256, 16/2, 8 rows 7.9 / 9.8, 17 rows 9.0 / 10.6, 32 rows
+// 12.2 / 12.2)
+__host__ __device__ constexpr int hd_min_rows(int D) { return D == 256 ? 24 : 16; }
 
 struct PrefillHdParams {
     uint16_t* out;
@@ -104,19 +110,20 @@ __device__ __forceinline__ int hd_wave_max(int v) {
     return __builtin_amdgcn_readfirstlane(v);
 }
 
-template <int D, bool BF>
-__global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
+template <int D, bool BF, int W>
+__global__ void __launch_bounds__(64 * W, D == 256 && W == 4 ? 1 : 2) prefill_hd_kernel(PrefillHdParams p) {
     using M = MT<BF>;
     using V8 = typename M::v8;
     constexpr int NS = D == 256 ? 2 : 3;        // tile slots
     constexpr int ROW = 2 * D, TILE = kHdBN * ROW;
-    constexpr int NTR = TILE / (1024 * kHdW);   // transfers per wave and tensor
+    constexpr int NTR = TILE / (1024 * W);      // transfers per wave and tensor
     constexpr int NTERM = WeightTerms<BF>::n;   // 16-bit terms of a weight
     constexpr int HB = D == 256 ? 1 : 2;        // 32-key blocks per softmax round
+    constexpr int KA = D == 256 && W == 4 ? 6 : 2, VA = D == 256 && W == 4 ? 4 : 1;  // operand reads ahead
     constexpr float kOff = BF ? 0.0f : 7.0f;    // weights are 2^(s - m + kOff), at most 2^15
     struct Lds {
         uint8_t tile[NS][2][TILE];  // [slot][K, V]
-        float qs[kHdW][D];          // rows that rerun key by key
+        float qs[W][D];             // rows that rerun key by key
     };
     __shared__ __attribute__((aligned(1024))) Lds lds;
 
@@ -167,8 +174,7 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
         }
     }
 
-    // ---- tile transfers: wave w fills rows 8w .. 8w + 7, 1 KB (2 or 8 rows) at
-    // a time; lane L's 16 bytes land at position L of that KB
+    // ---- tile transfers: wave w fills 64 / W rows, 1 KB (2 or 8 rows) at a time; lane L's 16 bytes land at position L of that KB
     const int64_t row_stride = (int64_t)p.Hkv * ROW;  // bytes between keys
     const uint8_t* kg = reinterpret_cast<const uint8_t*>(p.k) + (int64_t)g * ROW;
     const uint8_t* vg = reinterpret_cast<const uint8_t*>(p.v) + (int64_t)g * ROW;
@@ -176,7 +182,7 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
     uint32_t tr_col[NTR];
 #pragma unroll
     for (int i = 0; i < NTR; ++i) {
-        tr_row[i] = 8 * w + i * (1024 / ROW) + lane / (D / 8);
+        tr_row[i] = kHdBN / W * w + i * (1024 / ROW) + lane / (D / 8);
         tr_col[i] = 16u * (uint32_t)((lane % (D / 8)) ^ hd_tile_swz<D>(tr_row[i]));
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
@@ -243,21 +249,21 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
             // one.  Fixed by scheduling barriers: left alone, the compiler
             // issues each read right before the product that waits for it (593
             // against 565 us on the 4 prompts named above, with the store).
-            u32x4 ka[3][HB];
+            u32x4 ka[KA + 1][HB];
             auto read_k = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
                 for (int b = 0; b < HB; ++b)
-                    ka[s % 3][b] = lds128((k_slot ^ (uint32_t)(32 * (s & 7))) +
+                    ka[s % (KA + 1)][b] = lds128((k_slot ^ (uint32_t)(32 * (s & 7))) +
                                           (uint32_t)((HB * r + b) * 32 * ROW + 256 * (s >> 3)));
             };
-            read_k(0);
-            read_k(1);
+#pragma unroll
+            for (int s = 0; s < KA; ++s) read_k(s);
 #pragma unroll
             for (int s = 0; s < D / 16; ++s) {
-                if (s + 2 < D / 16) read_k(s + 2);
+                if (s + KA < D / 16) read_k(s + KA);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int b = 0; b < HB; ++b) sacc[b] = M::mma(as_v8<V8>(ka[s % 3][b]), qf[s], sacc[b]);
+                for (int b = 0; b < HB; ++b) sacc[b] = M::mma(as_v8<V8>(ka[s % (KA + 1)][b]), qf[s], sacc[b]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (need_mask) {
@@ -304,22 +310,24 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
                 }
             l_part += sum;
             // O^T += V^T P^T, V operands (two transposing reads each) one ahead
-            u32x2 va[2][2];
+            u32x2 va[VA + 1][2];
             auto read_v = [&](int i) __attribute__((always_inline)) {
                 const int c = i / (D / 32), m = i % (D / 32);
                 const int vo = (2 * HB * r + c) * 16 * ROW + 256 * (m >> 2);
 #pragma unroll
                 for (int sec = 0; sec < 2; ++sec)
-                    va[i & 1][sec] = lds_tr((v_slot[sec] ^ (uint32_t)(64 * (m & 3))) + (uint32_t)vo);
+                    va[i % (VA + 1)][sec] = lds_tr((v_slot[sec] ^ (uint32_t)(64 * (m & 3))) + (uint32_t)vo);
             };
             constexpr int NV = 2 * HB * (D / 32);
-            read_v(0);
+#pragma unroll
+            for (int i = 0; i < VA; ++i) read_v(i);
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
-                if (i + 1 < NV) read_v(i + 1);
+                if (i + VA < NV) read_v(i + VA);
                 __builtin_amdgcn_sched_barrier(0);
                 const int c = i / (D / 32), m = i % (D / 32);
-                const V8 x = as_v8<V8>(u32x4{va[i & 1][0][0], va[i & 1][0][1], va[i & 1][1][0], va[i & 1][1][1]});
+                const u32x2* vi = va[i % (VA + 1)];
+                const V8 x = as_v8<V8>(u32x4{vi[0][0], vi[0][1], vi[1][0], vi[1][1]});
 #pragma unroll
                 for (int u = 0; u < NTERM; ++u) o[m] = M::mma(x, as_v8<V8>(pt[u][c]), o[m]);
                 __builtin_amdgcn_sched_barrier(0);
@@ -378,15 +386,18 @@ __global__ void __launch_bounds__(512, 2) prefill_hd_kernel(PrefillHdParams p) {
     }
 }
 
-template <int D>
-int launch_prefill_hd(const PrefillHdParams& prm, bool bf, unsigned grid, hipStream_t s) {
-    if (bf) hipLaunchKernelGGL((prefill_hd_kernel<D, true>), dim3(grid), dim3(64 * kHdW), 0, s, prm);
-    else hipLaunchKernelGGL((prefill_hd_kernel<D, false>), dim3(grid), dim3(64 * kHdW), 0, s, prm);
+template <int W>
+int launch_prefill_hd(const PrefillHdParams& prm, int D, bool bf, hipStream_t s) {
+    const dim3 grid((unsigned)((int64_t)prm.ntiles * prm.Hkv * prm.hgroups)), block(64 * W);
+    if (D == 64 && bf) hipLaunchKernelGGL((prefill_hd_kernel<64, true, W>), grid, block, 0, s, prm);
+    else if (D == 64) hipLaunchKernelGGL((prefill_hd_kernel<64, false, W>), grid, block, 0, s, prm);
+    else if (bf) hipLaunchKernelGGL((prefill_hd_kernel<256, true, W>), grid, block, 0, s, prm);
+    else hipLaunchKernelGGL((prefill_hd_kernel<256, false, W>), grid, block, 0, s, prm);
     VMC_LAUNCH_CHECK();
     return VMC_OK;
 }
 
-PrefillHdParams hd_params(const GenArgs& a) {
+PrefillHdParams hd_params(const GenArgs& a, int waves) {
     PrefillHdParams prm = {};
     prm.out = reinterpret_cast<uint16_t*>(a.out);
     prm.q = reinterpret_cast<const uint16_t*>(a.q);
@@ -398,9 +409,9 @@ PrefillHdParams hd_params(const GenArgs& a) {
     prm.Hkv = a.Hkv;
     prm.G = a.Hq / a.Hkv;
     prm.scale = a.scale;
-    // heads per workgroup: 4, 2 or 1, dividing G; 32-row blocks per head fill 8 waves
+    // heads per workgroup: 4, 2 or 1, dividing G; 32-row blocks per head fill the waves
     prm.hw = prm.G % 4 == 0 ? 4 : (prm.G % 2 == 0 ? 2 : 1);
-    prm.rb = kHdW / prm.hw;
+    prm.rb = waves / prm.hw;
     prm.qb = 32 * prm.rb;
     prm.hgroups = prm.G / prm.hw;
     prm.ntiles = (a.rows - 1) / prm.qb + 1;
@@ -410,18 +421,26 @@ PrefillHdParams hd_params(const GenArgs& a) {
 }  // namespace
 
 bool prefill_hd_takes(const GenArgs& a) {
-    if (a.src != GEN_LOCAL || (a.D != 64 && a.D != 256) || a.rows <= 0 || a.rows > 0x7fffffff - 1024) return false;
-    const PrefillHdParams prm = hd_params(a);
+    if (a.src != GEN_LOCAL || (a.D != 64 && a.D != 256) || a.rows <= hd_min_rows(a.D) || a.rows > 0x7fffffff - 1024)
+        return false;
+    const PrefillHdParams prm = hd_params(a, 8);
     return (int64_t)prm.ntiles * prm.Hkv * prm.hgroups <= 0x7fffffff &&
            (int64_t)kHdBN * a.Hkv * 2 * a.D <= 0x7fffffff &&  // a tile's 32-bit offsets
            (((uintptr_t)a.q | (uintptr_t)a.out | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0;
 }
 
 int prefill_hd(const GenArgs& a, hipStream_t s) {
-    const PrefillHdParams prm = hd_params(a);
-    const unsigned grid = (unsigned)((int64_t)prm.ntiles * prm.Hkv * prm.hgroups);
-    return a.D == 64 ? launch_prefill_hd<64>(prm, a.q_bf16 != 0, grid, s)
-                     : launch_prefill_hd<256>(prm, a.q_bf16 != 0, grid, s);
+    // Four waves while their workgroups fit the CUs, one each at head_dim 256
+    // (128 KB of tiles) and four at 64: shorter blocks see fewer tiles of their
+    // neighbours' keys, and half as many waves load, multiply and store on a CU.
+    // bf16, us for eight waves / four: 256, 16/2 heads, 8 prompts of 20 tokens 20.0
+    // / 14.8, one of 1000 90.5 / 76.6 (past the line: 8 of 500 62 / 86); 64, 32/8,
+    // 8 of 20 10.0 / 6.4, one of 4096 197 / 170 (past the line: one of 8000 555 /
+    // 575).
+    const PrefillHdParams half = hd_params(a, 4);
+    if ((int64_t)half.ntiles * half.Hkv * half.hgroups <= (int64_t)num_cus() * (a.D == 64 ? 4 : 1))
+        return launch_prefill_hd<4>(half, a.D, a.q_bf16 != 0, s);
+    return launch_prefill_hd<8>(hd_params(a, 8), a.D, a.q_bf16 != 0, s);
 }
 
 }  // namespace vmc
