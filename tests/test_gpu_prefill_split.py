@@ -91,3 +91,39 @@ def test_paged(dev, fmt, heads):
         return out
 
     _close(run(1), run(reps)[:t], bf16)
+
+
+# one block of rows and one head a workgroup (128 rows or fewer: the keys stay
+# whole over this step's K/V and 4-bit values), and one row more, against fp64;
+# tolerance as the oracle comparisons of the two paths
+@pytest.mark.parametrize("t", [1, 33, 128, 129])
+@pytest.mark.parametrize("fmt", [None, "turboquant_4bit_nc", "turboquant_3bit_nc"])
+def test_one_block(dev, fmt, t):
+    import torch
+    from kvgen import close_report
+    from vm_c_amd import capi
+    hq, hkv, prefix = 7, 1, 0 if fmt is None else 300
+    t = max(t, 17) if fmt else t  # shorter steps over slots take decode rows
+    w = make_workload([prefix + t], Hq=hq, Hkv=hkv, seed=t)
+    K, V = (torch.from_numpy(x.astype(np.float32)).to(dev).half() for x in (w.K, w.V))
+    pos = torch.arange(prefix, prefix + t, dtype=torch.int32, device=dev)
+    q = torch.randn(t, hq, 128, generator=torch.Generator(device=dev).manual_seed(6), device=dev).half()
+    out = torch.full_like(q, float("nan"))
+    bits = lambda x: np.ascontiguousarray(x.cpu().numpy().view(np.uint16))  # noqa: E731
+    if fmt is None:
+        capi.flash_attention_prefill(out, q, K, V, pos, hkv, float(w.scale))
+        ex = O.prefill_exact_rows(bits(q), bits(K), bits(V), np.asarray([0, t]), hkv, float(w.scale),
+                                  np.repeat(np.arange(t), hq), np.tile(np.arange(hq), t), is_bf16=False)
+    else:
+        cfg, L = capi.tq_config(128, fmt), O.tq_layout(fmt)
+        cache = torch.zeros(w.num_blocks * BS * hkv * cfg.slot_size_aligned, dtype=torch.uint8, device=dev)
+        capi.turboquant_store(K, V, cache, torch.from_numpy(w.slots).to(dev), BS, cfg)
+        capi.turboquant_prefill_attention(out, q, cache, torch.from_numpy(w.bt).to(dev),
+                                          torch.zeros(t, dtype=torch.int32, device=dev), pos, hkv, float(w.scale), cfg,
+                                          block_size=BS)
+        c, _ = O.tq_tables(128, cfg.key_quant_bits)
+        ex = O.tq_decode_exact(bits(q), cache.cpu().numpy(), np.repeat(w.bt, t, 0), pos.cpu().numpy() + 1, hkv,
+                               float(w.scale), BS, L, c, bf16=False)
+    torch.cuda.synchronize()
+    ok, err = close_report(out.float().cpu().numpy().reshape(ex.shape), ex, 2e-3, 1e-2)
+    assert ok, f"max err {err}"

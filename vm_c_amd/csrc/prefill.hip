@@ -86,8 +86,9 @@ size_t vt_workspace_bytes(int64_t num_tokens, int64_t num_kv_heads) {
     return (size_t)(n * (kD * BN * 2) + ((n + 255) & ~(int64_t)255));
 }
 
-// workgroup shape shared by the local and paged entry points
-void set_tiling(PrefillParams& prm, int num_tokens, int num_heads, int num_kv_heads, float scale) {
+// workgroup shape shared by the local and paged entry points; whole_alone: see
+// the rule at the end
+void set_tiling(PrefillParams& prm, int num_tokens, int num_heads, int num_kv_heads, float scale, bool whole_alone) {
     prm.T = num_tokens;
     prm.Hq = num_heads;
     prm.Hkv = num_kv_heads;
@@ -111,7 +112,15 @@ void set_tiling(PrefillParams& prm, int num_tokens, int num_heads, int num_kv_he
     // 101; 3-bit slots 512 201 / 168; a 1024-token prompt 39 / 32).  Past
     // that the workgroups take turns and each tile is fetched twice as often
     // (q8_0 1536 tokens 205 / 252, 2048 245 / 281).
-    if (shape(2) > num_cus()) shape(1);
+    // No more workgroups come of it where one block holds all rows, and with one
+    // head a workgroup the four waves of 128 rows already sit on four SIMDs:
+    // over this step's K/V and over slots with 4-bit values the second wave then
+    // costs more than it brings (28/4 heads, us for one wave / two: a 64-token
+    // prompt 6.1 / 7.0; 64 tokens over a 4096-token prefix, 4-bit slots 157 / 172,
+    // 3/4-bit 153 / 168, k8v4 207 / 225; but 3-bit slots of 100 tokens 160 / 152,
+    // q8_0 of 64 107 / 100, fp16 96 / 85).
+    const int64_t split = shape(2);
+    if (split > num_cus() || (whole_alone && prm.hw == 1 && prm.ntiles == 1)) shape(1);
 }
 
 int launch_tiled(PrefillParams& prm, bool bf16, int fmt, int src, bool vt, hipStream_t s) {
@@ -137,7 +146,7 @@ int tq_prefill_tiled(void* out, const void* query, const void* kv_cache, const i
     prm.out = reinterpret_cast<uint16_t*>(out);
     prm.q = reinterpret_cast<const uint16_t*>(query);
     prm.pos = token_positions;
-    set_tiling(prm, num_tokens, num_heads, num_kv_heads, scale);
+    set_tiling(prm, num_tokens, num_heads, num_kv_heads, scale, cfg->value_quant_bits == 4);
     prm.kp = prm.vp = reinterpret_cast<const uint8_t*>(kv_cache);
     prm.bt = block_tables;
     prm.tok_seq = token_to_seq;
@@ -234,7 +243,7 @@ extern "C" int vmc_flash_attention_prefill_v2(void* output, const void* query, c
     prm.out = reinterpret_cast<uint16_t*>(output);
     prm.q = reinterpret_cast<const uint16_t*>(query);
     prm.pos = token_positions;
-    set_tiling(prm, num_tokens, num_heads, num_kv_heads, scale);
+    set_tiling(prm, num_tokens, num_heads, num_kv_heads, scale, false);
     prm.kp = reinterpret_cast<const uint8_t*>(key_cache);
     prm.vp = reinterpret_cast<const uint8_t*>(value_cache);
     prm.bt = block_tables;
@@ -314,7 +323,7 @@ int local_prefill(void* output, const void* query, const void* key, const void* 
     prm.k = reinterpret_cast<const uint16_t*>(key);
     prm.v = reinterpret_cast<const uint16_t*>(value);
     prm.pos = token_positions;
-    set_tiling(prm, num_tokens, num_heads, num_kv_heads, scale);
+    set_tiling(prm, num_tokens, num_heads, num_kv_heads, scale, true);
     int fmt = -1;
     if (key_cache) {
         const int64_t E = vmc_kv_entry_bytes(kv_format, head_dim);
