@@ -1,9 +1,11 @@
 """Causal prefill parity on the GPU: HIP MFMA prefill vs exact fp64 causal
 attention (oracle), tolerance |got - ref| <= 2e-3 + 1e-2 |ref|; the fused
 quantize-on-append must write the same bytes as the standalone append.  Each
-case runs through vmc_flash_attention_prefill and, with a workspace of
-prebuilt V^T tiles, through vmc_flash_attention_prefill_ws, whose outputs
-must equal the first's bit for bit wherever neither runs the exact mode."""
+case runs through vmc_flash_attention_prefill and, with a workspace (of prebuilt
+V^T tiles in bf16), through vmc_flash_attention_prefill_ws, whose bf16 outputs
+must equal the first's bit for bit wherever neither runs the exact mode.  Short
+steps split a tile's keys between two waves; the cases of the append and of the
+exact mode also run in steps long enough that they do not (LONG)."""
 import os
 
 import numpy as np
@@ -15,6 +17,9 @@ from kvgen import BS, close_report, crc, prefill_inputs
 pytestmark = pytest.mark.gpu
 
 ATOL, RTOL = 2e-3, 1e-2
+# sequences that bring a step of 8 / 2 heads past 4096 tokens, i.e. past 256
+# workgroups of 32 rows x 4 heads
+LONG = [720] * 6
 
 
 def _inputs(seq_lens, Hq, Hkv, D=128, seed=0, bf16=True):
@@ -71,21 +76,29 @@ def _slots_for(T, seed):
     return perm[t // BS] * BS + t % BS, nblk
 
 
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("more", [[], LONG])
 @pytest.mark.parametrize("ws", [False, True])
 @pytest.mark.parametrize("fmt", [O.KV_Q8_0, O.KV_Q4_0, O.KV_F16, O.KV_BF16])
-def test_prefill_fused_append_bitexact(dev, fmt, ws):
-    seq_lens, Hq, Hkv = [333, 190], 8, 2
-    qb, kb, vb, pos, cu = _inputs(seq_lens, Hq, Hkv, seed=13)
+def test_prefill_fused_append_bitexact(dev, fmt, ws, more, bf16):
+    seq_lens, Hq, Hkv = [333, 190] + more, 8, 2
+    qb, kb, vb, pos, cu = _inputs(seq_lens, Hq, Hkv, seed=13, bf16=bf16)
     T = qb.shape[0]
     slots, nblk = _slots_for(T, 3)
     slots[7] = -1
     E = O.entry_bytes(fmt, 128)
     nbytes = nblk * BS * Hkv * E
-    got, kc, vc = _run(dev, qb, kb, vb, pos, Hkv, 1.0 / np.sqrt(128), append=(fmt, slots, nbytes), ws=ws)
+    got, kc, vc = _run(dev, qb, kb, vb, pos, Hkv, 1.0 / np.sqrt(128), bf16=bf16, append=(fmt, slots, nbytes), ws=ws)
     kr = np.zeros(nbytes, np.uint8)
     vr = np.zeros(nbytes, np.uint8)
-    O.kv_append(kb, vb, slots, kr, vr, BS, fmt, src_bf16=True)
+    O.kv_append(kb, vb, slots, kr, vr, BS, fmt, src_bf16=bf16)
     assert np.array_equal(kc, kr) and np.array_equal(vc, vr)
+    # the attention beside the append: every head of some tokens
+    toks = np.repeat(np.unique(np.r_[0:T:97, T - 1, cu[1:-1]]), Hq)
+    heads = np.tile(np.arange(Hq), len(toks) // Hq)
+    ex = O.prefill_exact_rows(qb, kb, vb, cu, Hkv, 1.0 / np.sqrt(128), toks, heads, is_bf16=bf16)
+    ok, err = close_report(got[toks, heads], ex, ATOL, RTOL)
+    assert ok, f"max err {err}"
 
 
 def test_prefill_config4_full_size(dev):
@@ -126,8 +139,9 @@ def test_prefill_config4_full_size(dev):
     assert np.array_equal(kc, kr) and np.array_equal(vc, vr)
 
 
+@pytest.mark.parametrize("more", [[], LONG])
 @pytest.mark.parametrize("ws", [False, True])
-def test_prefill_bf16_v_outside_fp16_range(dev, ws):
+def test_prefill_bf16_v_outside_fp16_range(dev, ws, more):
     """bf16 V that fp16 cannot hold: one sequence at 2^100 scale (fp16
     overflows), one at 2^-20 (fp16 subnormals keep 4 bits) with bf16
     subnormals mixed in, one N(0,1) with sparse +-1e30 and +-1e-38 spikes
@@ -137,7 +151,7 @@ def test_prefill_bf16_v_outside_fp16_range(dev, ws):
     attention after dividing both by the sequence's magnitude, so the usual
     tolerance is relative to that scale."""
     from kvgen import f32_to_bf16_bits
-    seq_lens, Hq, Hkv = [300, 77, 129, 200], 8, 2
+    seq_lens, Hq, Hkv = [300, 77, 129, 200] + more, 8, 2
     qb, kb, _, pos, cu = _inputs(seq_lens, Hq, Hkv, seed=21)
     T = qb.shape[0]
     rng = np.random.default_rng(22)
@@ -167,34 +181,37 @@ def test_prefill_bf16_v_outside_fp16_range(dev, ws):
         assert ok, f"sequence {b}: max scaled err {err}"
 
 
-@pytest.mark.parametrize("bf16", [True, False])
 @pytest.mark.parametrize("seq_lens,Hq,Hkv", [([256, 512, 64, 128], 8, 2), ([300, 77, 129], 4, 1),
-                                              ([1000, 24], 32, 8)])
-def test_prefill_ws_equals_in_kernel_transpose(dev, bf16, seq_lens, Hq, Hkv):
-    """Prebuilt V^T tiles (sequences starting on 64-key boundaries) and the
+                                              ([1000, 24], 32, 8), ([256, 512, 64, 128, 300] + LONG, 8, 2)])
+def test_prefill_ws_equals_in_kernel_transpose(dev, seq_lens, Hq, Hkv):
+    """bf16: prebuilt V^T tiles (sequences starting on 64-key boundaries) and the
     in-kernel pass (the others) give the same bits."""
-    qb, kb, vb, pos, cu = _inputs(seq_lens, Hq, Hkv, seed=31, bf16=bf16)
+    qb, kb, vb, pos, cu = _inputs(seq_lens, Hq, Hkv, seed=31)
     scale = 1.0 / np.sqrt(128)
-    a = _run(dev, qb, kb, vb, pos, Hkv, scale, bf16=bf16)
-    b = _run(dev, qb, kb, vb, pos, Hkv, scale, bf16=bf16, ws=True)
+    a = _run(dev, qb, kb, vb, pos, Hkv, scale)
+    b = _run(dev, qb, kb, vb, pos, Hkv, scale, ws=True)
     assert np.isfinite(a).all()
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-def test_prefill_ws_fp16_inf_in_a_shared_tile(dev):
+@pytest.mark.parametrize("ws", [False, True])
+def test_prefill_fp16_inf_in_a_shared_tile(dev, ws):
     """fp16 V with an inf in the second sequence, which shares a 64-key tile
-    with the first: the tile's flag sends the workgroups that read it to
-    the in-kernel pass, so the two paths agree bit for bit; the first
-    sequence's rows of other tiles and the third sequence (no shared tile)
-    stay finite.  (Rows whose tile holds the inf, masked or not, are not
-    finite on either path: 0 * inf in the P . V product.)"""
+    with the first: the first sequence's rows of the other tile, the third
+    sequence (no shared tile) and the other KV head's query heads are right,
+    with and without a workspace (which fp16 steps check and leave alone).  A
+    row whose tile holds the inf, masked or not, is not finite: 0 * inf in the
+    P . V product."""
     seq_lens, Hq, Hkv = [100, 28, 64], 8, 2
     qb, kb, vb, pos, cu = _inputs(seq_lens, Hq, Hkv, seed=33, bf16=False)
+    scale = 1.0 / np.sqrt(128)
+    T = qb.shape[0]
+    toks, heads = np.repeat(np.arange(T), Hq), np.tile(np.arange(Hq), T)
+    ex = O.prefill_exact_rows(qb, kb, vb, cu, Hkv, scale, toks, heads, is_bf16=False).reshape(T, Hq, 128)
     vb = vb.copy()
     vb[cu[1] + 3, 1, 17] = 0x7C00  # +inf, second sequence, KV head 1
-    scale = 1.0 / np.sqrt(128)
-    a = _run(dev, qb, kb, vb, pos, Hkv, scale, bf16=False)
-    b = _run(dev, qb, kb, vb, pos, Hkv, scale, bf16=False, ws=True)
-    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
-    assert np.isfinite(b[:64]).all() and np.isfinite(b[cu[2]:cu[3]]).all()
-    assert np.isfinite(b[cu[0]:cu[1], :4]).all()  # query heads of KV head 0
+    got = _run(dev, qb, kb, vb, pos, Hkv, scale, bf16=False, ws=ws)
+    for rows, hs in ((slice(0, 64), slice(None)), (slice(cu[2], cu[3]), slice(None)), (slice(None), slice(0, 4))):
+        ok, err = close_report(got[rows, hs], ex[rows, hs], ATOL, RTOL)
+        assert ok, f"max err {err}"
+    assert not np.isfinite(got[cu[1] + 3:cu[2], 4:, 17]).any()
