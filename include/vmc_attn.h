@@ -110,10 +110,12 @@ int vmc_convert_fp8(void* dst_cache, const void* src_cache, double scale, int64_
  * sequences).  head_dim 64 and 256 with block_size 16, num_heads /
  * num_kv_heads <= 16, 16-byte aligned operands and f16 / bf16 pages of
  * q_dtype or GGUF pages run the MFMA decode: the same two launches where the
- * workspace has room for partial rows, else one pass per sequence.  Other
- * shapes run a one-wave-per-row kernel
- * (one launch, no workspace).  No host synchronisation.  The workspace size
- * depends on the current device's CU count.
+ * workspace has room for partial rows, else (without one, from 1024 rows on
+ * and where max_num_blocks_per_req is 4 or less, at head_dim 64 8) one pass
+ * per sequence.  Other shapes run a one-wave-per-row kernel (one launch, no
+ * workspace).  No host synchronisation.  The workspace size depends on the
+ * current device's CU count.  Concurrent calls on one workspace race, at
+ * head_dim 64 and 256 too: two streams need one each.
  */
 size_t vmc_paged_decode_workspace_size(int batch_size, int num_heads, int num_kv_heads,
                                        int head_dim, int max_num_blocks_per_req, int block_size,

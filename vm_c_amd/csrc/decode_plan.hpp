@@ -20,7 +20,7 @@ struct DecodeParams {
     const uint8_t* vc;
     const int32_t* bt;
     const int32_t* seq_lens;
-    float* part;  // [2 * grid][Hq][D + 2]: o, m, l of cut sequences
+    float* part;  // [2 * grid][Hq][D + 4]: o, m, l, 2 unused, of cut sequences
     int B, Hq, Hkv, G, max_blocks;
     float scale_log2;
     int64_t page_bytes;  // one page of one cache, all heads
