@@ -451,7 +451,12 @@ __global__ void __launch_bounds__(1024) decode_merge_kernel(DecodeParams p) {
 // one load of 64 lengths after another, 1000 rows of up to 300 keys (14 / 2
 // heads of 64, bf16) took 99 us with their split pass, now 71 (8 / 1 heads of 256:
 // 105, 83).
-template <int D>
+// PAGES: the pages' decode.  The TurboQuant decode of 256 dims goes without the
+// look for pieces of weight 0 (its values are codes times 16-bit scales) and with
+// one head a workgroup, grid (B, Hq): the selects and the loop over heads break
+// up a round's loads (4 sequences of up to 32768 tokens, 8/1 heads, split pass
+// and merge: 50 us with them, 43 without).
+template <int D, bool PAGES>
 __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) {
     constexpr int NV = D / 64;
     static_assert(NV == 1 || NV == 4, "head_dim 64 or 256");
@@ -460,17 +465,18 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
     const int b = blockIdx.x;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int carry = 0, ps_b = 0, pg_b = 0;
-    for (int b0 = 0; b0 < p.B; b0 += 256) {
-        int pgs[4] = {};
+    constexpr int NU = PAGES ? 4 : 1;
+    for (int b0 = 0; b0 < p.B; b0 += 64 * NU) {
+        int pgs[NU] = {};
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {  // four loads in flight
+        for (int u = 0; u < NU; ++u) {
             int L = 0;
             if (u > 0 && b0 + 64 * u >= p.B) break;  // uniform
-            const int r = b0 + 64 * u + lane, n = seq_pages(p, min(r, p.B - 1), &L);
-            pgs[u] = r < p.B ? n : 0;
+            const int r = b0 + 64 * u + lane;
+            pgs[u] = r < p.B ? seq_pages(p, r, &L) : 0;
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < NU; ++u) {
             const int bu = b0 + 64 * u;
             if (bu >= p.B) break;  // uniform
             const int incl = wave_incl_scan(pgs[u], lane);
@@ -501,8 +507,9 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
     if (w0 == w1) return;  // written by its range
     const int nseg = w1 - w0 + 1;
     const int64_t rs = (int64_t)p.Hq * (D + 4);
-    for (int hq = blockIdx.y; hq < p.Hq; hq += gridDim.y) {
-        if (hq != (int)blockIdx.y) __syncthreads();  // the last head's sums are read
+    int hq = blockIdx.y;
+    do {
+        if (PAGES && hq != (int)blockIdx.y) __syncthreads();  // the last head's sums are read
         auto row = [&](int s) {  // piece s = range w0 + s
             const int64_t slot = s == 0 ? 2 * w0 + 1 : 2 * (w0 + s);
             return p.part + slot * rs + (int64_t)hq * (D + 4);
@@ -523,7 +530,7 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
             for (int u = 0; u < 16; ++u) mx = s0 + 4 * u < nseg ? fmaxf(mx, ml[u].x) : mx;
             if (mx > M && M != kNegInf) {  // wave-uniform
                 const float f = __builtin_amdgcn_exp2f(M - mx);
-                const bool none = f == 0.0f && L == L;
+                const bool none = PAGES && f == 0.0f && L == L;
                 L *= f;
 #pragma unroll
                 for (int e = 0; e < NV; ++e) acc[e] = none ? 0.0f : acc[e] * f;
@@ -533,7 +540,7 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
                 const float wu = s0 + 4 * u < nseg ? __builtin_amdgcn_exp2f(ml[u].x - Mu) : 0.0f;
-                const bool none = wu == 0.0f && ml[u].y == ml[u].y;
+                const bool none = PAGES && wu == 0.0f && ml[u].y == ml[u].y;
                 L = __builtin_fmaf(ml[u].y, wu, L);
 #pragma unroll
                 for (int e = 0; e < NV; ++e) acc[e] = __builtin_fmaf(none ? 0.0f : o[u][e], wu, acc[e]);
@@ -555,7 +562,7 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             const float f = red[w][D] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(red[w][D] - Mgu);
-            const bool none = f == 0.0f && red[w][D + 1] == red[w][D + 1];
+            const bool none = PAGES && f == 0.0f && red[w][D + 1] == red[w][D + 1];
             Lg = __builtin_fmaf(red[w][D + 1], f, Lg);
             const fv v = *reinterpret_cast<const fv*>(&red[w][NV * lane]);
 #pragma unroll
@@ -565,7 +572,7 @@ __global__ void __launch_bounds__(256) decode_merge_rows_kernel(DecodeParams p) 
 #pragma unroll
         for (int e = 0; e < NV; ++e) og[e] *= inv;
         put(hq, og);
-    }
+    } while (PAGES && (hq += gridDim.y) < p.Hq);
 }
 
 }  // namespace

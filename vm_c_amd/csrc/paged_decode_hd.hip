@@ -473,7 +473,7 @@ int launch_hd(DecodeParams& prm, hipStream_t stream) {
                        stream, prm);
     VMC_LAUNCH_CHECK();
     if (!prm.per_seq) {
-        hipLaunchKernelGGL(decode_merge_rows_kernel<D>, dim3(prm.B, merge_rows_y(prm.B, prm.Hq)), dim3(256), 0,
+        hipLaunchKernelGGL((decode_merge_rows_kernel<D, true>), dim3(prm.B, merge_rows_y(prm.B, prm.Hq)), dim3(256), 0,
                            stream, prm);
         VMC_LAUNCH_CHECK();
     }

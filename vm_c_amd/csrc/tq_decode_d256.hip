@@ -584,8 +584,7 @@ int launch_d256(DecodeParams& prm, hipStream_t stream) {
     hipLaunchKernelGGL((tq_decode_d256_kernel<KB, HK, BF>), dim3(nwg), dim3(512), 0, stream, prm);
     VMC_LAUNCH_CHECK();
     if (!prm.per_seq) {
-        hipLaunchKernelGGL(decode_merge_rows_kernel<kD2>, dim3(prm.B, merge_rows_y(prm.B, prm.Hq)), dim3(256), 0,
-                           stream, prm);
+        hipLaunchKernelGGL((decode_merge_rows_kernel<kD2, false>), dim3(prm.B, prm.Hq), dim3(256), 0, stream, prm);
         VMC_LAUNCH_CHECK();
     }
     return VMC_OK;
